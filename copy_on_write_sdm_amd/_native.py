@@ -25,7 +25,7 @@ SOURCE_DIR = PACKAGE_DIR / "csrc"
 # one translation unit per step-kernel family so hipcc can run in parallel
 SOURCES = ("cowsdm.hip", "step_i32_packed.hip", "step_i32_dense.hip", "step_i64_packed.hip",
            "step_i64_dense.hip", "trace_plan.hip", "routes.hip", "controller.hip",
-           "recurrence.hip")
+           "recurrence.hip", "route_recurrence.hip")
 INCLUDE_DIR = REPO_DIR / "include"
 LIBRARY = PACKAGE_DIR / "lib" / "libcowsdm.so"
 BUILD_DIR = PACKAGE_DIR / "_build"
@@ -245,6 +245,30 @@ class Recurrence(ctypes.Structure):
     ]
 
 
+class RouteRecurrence(ctypes.Structure):
+    """cowsdm_route_recurrence_t."""
+
+    _fields_ = [
+        ("batch", ctypes.c_int64),
+        ("time", ctypes.c_int64),
+        ("heads", ctypes.c_int64),
+        ("slots", ctypes.c_int64),
+        ("width", ctypes.c_int64),
+        ("writes", ctypes.c_int64),
+        ("reads", ctypes.c_int64),
+        ("initial_memory", ctypes.c_void_p),
+        ("write_indices", ctypes.c_void_p),
+        ("write_weights", ctypes.c_void_p),
+        ("values", ctypes.c_void_p),
+        ("input_gate", ctypes.c_void_p),
+        ("forget_log_gate", ctypes.c_void_p),
+        ("read_indices", ctypes.c_void_p),
+        ("read_weights", ctypes.c_void_p),
+        ("readings", ctypes.c_void_p),
+        ("final_memory", ctypes.c_void_p),
+    ]
+
+
 class HandoffLayer(ctypes.Structure):
     """cowsdm_handoff_layer_t."""
 
@@ -296,6 +320,7 @@ SIGNATURES: dict[str, tuple] = {
         _I32, [ctypes.POINTER(Controller), _P, _P, _I64, _P, _P, _P, ctypes.POINTER(Controller),
                _P, _P, _P, _P, _P, _P, _I64, _I64, _P, _P, _P, _P, _P]),
     "cowsdm_recurrence_forward": (_I32, [ctypes.POINTER(Recurrence), _P]),
+    "cowsdm_route_recurrence_forward": (_I32, [ctypes.POINTER(RouteRecurrence), _P]),
     "cowsdm_dense_routes": (_I32, [_P, _P, _I32, _I64, _I64, _I64, _P, _P, _P]),
     "cowsdm_host_report_alloc": (
         _I32, [_I64, ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_void_p)]),

@@ -8,11 +8,10 @@ copy-on-write state (``_pack_prefill_layer``, inference.py:314-366;
 
 Every token of the prefix goes through the controller kernels at once
 (``prepare_sdm_step`` over B*T tokens: input norm, projections, gates, the
-two route selections), the routes are scattered into dense vectors
-(``dense_sparse_routes``), the layer's recurrence runs over the sequence
-(``gated_delta_recurrence``, csrc/recurrence.hip), and the readings go
-through the controller's finish (readings norm, output gate, output
-projection).  Float32; there is no CPU path.
+two route selections), the layer's recurrence runs over the sequence on
+those routes as they are (``route_recurrence``, csrc/route_recurrence.hip),
+and the readings go through the controller's finish (readings norm, output
+gate, output projection).  Float32; there is no CPU path.
 """
 
 from __future__ import annotations
@@ -24,7 +23,7 @@ import torch
 
 from .controller import SDMController, finish_sdm_step, prepare_sdm_step
 from .inference import FaithfulSDMDecodeState, pack_prefill_layers
-from .recurrence import dense_sparse_routes, gated_delta_recurrence
+from .recurrence import route_recurrence
 
 
 @dataclass
@@ -69,24 +68,8 @@ def prefill_sdm_layer(controller: SDMController, initial_memory: torch.Tensor,
     step = prepare_sdm_step(c, tokens.reshape(batch * time, 1, width))
     x = step.inputs            # rows (b * T + t) * H + h
 
-    def by_bank(t: torch.Tensor) -> torch.Tensor:
-        # token-major rows -> [B * H, T, ...], bank b * H + h
-        rest = t.shape[1:]
-        return (t.reshape(batch, time, heads, *rest).transpose(1, 2)
-                .reshape(batch * heads, time, *rest).contiguous())
-
-    write_routes = dense_sparse_routes(by_bank(x.write_weights), by_bank(x.write_indices), slots)
-    read_routes = dense_sparse_routes(by_bank(x.read_weights), by_bank(x.read_indices), slots)
-    start = (initial_memory.unsqueeze(0).expand(batch, -1, -1, -1)
-             .reshape(batch * heads, slots, head_width).contiguous())
-    readings, final = gated_delta_recurrence(start, write_routes, by_bank(x.values),
-                                             by_bank(x.input_gate), by_bank(x.forget_log_gate),
-                                             read_routes)
-    del write_routes, read_routes
-    # back to token-major rows for the controller's finish
-    per_token = (readings.reshape(batch, heads, time, head_width).transpose(1, 2)
-                 .reshape(batch * time * heads, head_width).contiguous())
-    out = finish_sdm_step(c, step, per_token)
+    readings, final = route_recurrence(initial_memory, x, batch, time)
+    out = finish_sdm_step(c, step, readings)
 
     def routed(t: torch.Tensor) -> torch.Tensor:
         return t.reshape(batch, time, heads, *t.shape[1:])

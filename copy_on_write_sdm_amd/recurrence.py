@@ -7,7 +7,8 @@ recurrence the reference runs for training and prefill
 the recurrence takes.
 
 Kernels: ``cowsdm_recurrence_forward`` and ``cowsdm_dense_routes``
-(csrc/recurrence.hip).  Float32 only; there is no CPU path (the reference
+(csrc/recurrence.hip), and for the prefill, which holds the sparse routes,
+``cowsdm_route_recurrence_forward`` (csrc/route_recurrence.hip).  Float32 only; there is no CPU path (the reference
 falls back to its serial torch loop off CUDA, this module raises).
 
 The prefill handoff uses the recurrence's final memory: ``pack_prefill_layer``
@@ -126,6 +127,34 @@ def sdm_recurrence(initial_memory: torch.Tensor, write_routes: torch.Tensor,
               "cowsdm_recurrence_forward")
     if return_states:
         return readings, final, states
+    return readings, final
+
+
+@torch.no_grad()
+def route_recurrence(initial_memory: torch.Tensor, inputs, batch: int,
+                     time: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """``gated_delta_recurrence`` for the routes a controller just selected,
+    without their dense vectors: ``inputs`` holds B * T * H token-major rows
+    (the ``SDMStepInputs`` of ``prepare_sdm_step`` on B * T tokens), and every
+    bank b * H + h starts from ``initial_memory[h]`` [H, N, D].  Returns the
+    readings [B * T * H, D] and the final memory [B * H, N, D]."""
+
+    heads, slots, width = initial_memory.shape
+    if slots > MAX_SLOTS:
+        raise ValueError("dense SDM training recurrence supports at most 1,024 slots")
+    m0 = initial_memory.contiguous()
+    readings = torch.empty_like(inputs.values)
+    final = torch.empty(batch * heads, slots, width, device=m0.device, dtype=torch.float32)
+    r = nat.RouteRecurrence()
+    r.batch, r.time, r.heads, r.slots, r.width = batch, time, heads, slots, width
+    r.writes, r.reads = inputs.write_indices.shape[1], inputs.read_indices.shape[1]
+    r.initial_memory = m0.data_ptr()
+    for name in ("write_indices", "write_weights", "values", "input_gate", "forget_log_gate",
+                 "read_indices", "read_weights"):
+        setattr(r, name, getattr(inputs, name).data_ptr())
+    r.readings, r.final_memory = readings.data_ptr(), final.data_ptr()
+    nat.check(nat.lib().cowsdm_route_recurrence_forward(r, nat.stream_handle(m0.device)),
+              "cowsdm_route_recurrence_forward")
     return readings, final
 
 

@@ -718,6 +718,39 @@ typedef struct cowsdm_recurrence {
  * (the reference's "at most 1,024 slots"). */
 int32_t cowsdm_recurrence_forward(const cowsdm_recurrence_t* recurrence, void* stream);
 
+/* One SDM layer's token-serial recurrence over sparse routes (float32,
+ * device, contiguous): the recurrence of cowsdm_recurrence_t for routes that
+ * a controller just selected, without their dense vectors, as
+ * SparseDeltaMemory.forward runs it over a prefix (sdm.py:1136-1262; the
+ * token's arithmetic sdm.py:464-529).  Rows are token-major: token t of
+ * batch row b and head h is row (b * T + t) * H + h.  Every bank b * H + h
+ * starts from initial_memory[h]; the erase gate is the input gate.  A row's
+ * slots must differ; an entry outside [0, N) is left out. */
+typedef struct cowsdm_route_recurrence {
+  int64_t batch;                /* B                                   */
+  int64_t time;                 /* T >= 1                              */
+  int64_t heads;                /* H                                   */
+  int64_t slots;                /* N <= 1024                           */
+  int64_t width;                /* D, a head's width                   */
+  int64_t writes;               /* W <= 32                             */
+  int64_t reads;                /* R <= 32                             */
+  const float* initial_memory;  /* [H, N, D]                           */
+  const int64_t* write_indices; /* [B * T * H, W]                      */
+  const float* write_weights;   /* [B * T * H, W]                      */
+  const float* values;          /* [B * T * H, D]                      */
+  const float* input_gate;      /* [B * T * H]                         */
+  const float* forget_log_gate; /* [B * T * H]                         */
+  const int64_t* read_indices;  /* [B * T * H, R]                      */
+  const float* read_weights;    /* [B * T * H, R]                      */
+  float* readings;              /* [B * T * H, D]                      */
+  float* final_memory;          /* [B * H, N, D]                       */
+} cowsdm_route_recurrence_t;
+
+/* Runs the recurrence of cowsdm_route_recurrence_t; COWSDM_ELIMIT for
+ * N > 1024 or more than 32 routes a row. */
+int32_t cowsdm_route_recurrence_forward(const cowsdm_route_recurrence_t* recurrence,
+                                        void* stream);
+
 /* Dense route vectors from sparse routes, sdm.py:162-172
  * (dense_sparse_routes): dense [rows, slots] = 0 except
  * dense[row, indices[row, k]] = weights[row, k] (the last k wins for a
