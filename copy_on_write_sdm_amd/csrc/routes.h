@@ -21,6 +21,7 @@
 #pragma once
 
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -242,6 +243,279 @@ __device__ __forceinline__ void product_key_route_row(
   }
 }
 
+// ---- One lane per row (sqrt(N) <= 32) --------------------------------------
+//
+// The same selection with every row in one lane's registers: sorting
+// networks over 64-bit keys, no cross-lane operation, no LDS.  What bounds
+// the selection is its instructions, not bytes: at N = 256, K = 16 a wave
+// per row issues 2,180 for one row, most of them to broadcast keys, a lane
+// per row 2,300 for 64 rows.  A compare-exchange of two keys is one
+// v_max_f64 and one v_min_f64, at the rate of 32-bit operations on this
+// device, so keys are doubles.  131,072 rows (wave per row -> lane per row):
+// N = 256 K = 16 166 -> 17 us, K = 4 127 -> 5.4; N = 1,024 K = 32
+// 445 -> 30 us, K = 24 423 -> 69.
+
+// A score as a positive finite double in route_key's order: the score's
+// order-preserving bits below a fixed exponent bit (infinities and NaN
+// patterns are ordered doubles like the others), with 29 bits left below
+// them for `code`, which breaks ties.
+__device__ __forceinline__ double route_pack(float v, uint32_t code) {
+  const uint32_t bits = __float_as_uint(v);
+  const uint32_t order = bits ^ (static_cast<uint32_t>(static_cast<int32_t>(bits) >> 31) |
+                                 0x80000000u);
+  return __hiloint2double(static_cast<int>((order >> 3) | 0x20000000u),
+                          static_cast<int>((order << 29) | code));
+}
+
+__device__ __forceinline__ float route_score(double key) {
+  const uint32_t order = (static_cast<uint32_t>(__double2hiint(key)) << 3) |
+                         (static_cast<uint32_t>(__double2loint(key)) >> 29);
+  return __uint_as_float(order ^ (~static_cast<uint32_t>(static_cast<int32_t>(order) >> 31) |
+                                  0x80000000u));
+}
+
+__device__ __forceinline__ uint32_t route_code(double key) {
+  return static_cast<uint32_t>(__double2loint(key)) & 0x1fffffffu;
+}
+
+constexpr double kRouteAbsent = 0.0;   // below every route_pack key
+
+// v_max_f64 and v_min_f64 themselves: the keys are never NaN, and fmax would
+// quiet each operand first.
+__device__ __forceinline__ double key_max(double a, double b) {
+#ifdef __HIP_DEVICE_COMPILE__
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+#else
+  return a > b ? a : b;
+#endif
+}
+
+__device__ __forceinline__ double key_min(double a, double b) {
+#ifdef __HIP_DEVICE_COMPILE__
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+#else
+  return a < b ? a : b;
+#endif
+}
+
+__device__ __forceinline__ void sort_pair(double& high, double& low) {
+  const double h = key_max(high, low);
+  low = key_min(high, low);
+  high = h;
+}
+
+// x, bitonic, into descending order
+template <int N>
+__device__ __forceinline__ void bitonic_clean(double* x) {
+#pragma unroll
+  for (int d = N / 2; d > 0; d /= 2) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      if ((i & d) == 0) sort_pair(x[i], x[i + d]);
+    }
+  }
+}
+
+// Batcher's odd-even merge sort (K. E. Batcher, Sorting networks and their
+// applications, 1968), descending
+template <int N>
+__device__ __forceinline__ void network_sort(double* x) {
+#pragma unroll
+  for (int p = 1; p < N; p *= 2) {
+#pragma unroll
+    for (int k = p; k >= 1; k /= 2) {
+#pragma unroll
+      for (int j = k % p; j + k < N; j += 2 * k) {
+#pragma unroll
+        for (int i = 0; i < k; ++i) {
+          if (i + j + k < N && (i + j) / (2 * p) == (i + j + k) / (2 * p)) {
+            sort_pair(x[i + j], x[i + j + k]);
+          }
+        }
+      }
+    }
+  }
+}
+
+// top (descending) becomes the K highest of top and `other` (descending, of
+// length M <= K), descending
+template <int K, int M>
+__device__ __forceinline__ void merge_top(double* top, const double* other) {
+#pragma unroll
+  for (int i = 0; i < M; ++i) top[K - 1 - i] = key_max(top[K - 1 - i], other[i]);
+  bitonic_clean<K>(top);
+}
+
+// The K highest of x[0 .. N), descending, in x[0 .. K).
+template <int N, int K>
+__device__ __forceinline__ void network_top(double* x) {
+  if constexpr (N <= K) {
+    network_sort<N>(x);
+  } else {
+    network_top<N / 2, K>(x);
+    network_top<N / 2, K>(x + N / 2);
+    merge_top<K, K>(x, x + N / 2);
+  }
+}
+
+constexpr int route_pow2(int n) {
+  int p = 1;
+  while (p < n) p *= 2;
+  return p;
+}
+
+// Row `projected` ([2 * root], root <= NR) of the calling lane: its final_k
+// <= KP routes at weights and indices (`on` false: read, not written).
+// FULL: root == NR, sub == min(KP, NR), final_k == KP, and `projected` is
+// 16-byte aligned.
+template <int NR, int KP, bool FULL>
+__device__ __forceinline__ void product_key_route_lane(bool on,
+                                                       const float* __restrict__ projected,
+                                                       int root, int sub, int final_k,
+                                                       float* __restrict__ weights,
+                                                       int64_t* __restrict__ indices) {
+  constexpr int KL = KP < NR ? KP : NR;   // entries of a shortlist
+  if constexpr (FULL) {
+    root = NR;
+    sub = KL;
+    final_k = KP;
+  }
+  // 1. shortlists: score and index of the sub best of each half; the codes
+  // of lower positions are higher
+  float fv[KL], sv[KL];
+  uint32_t fi[KL], si[KL];
+  auto shortlist = [&](const float* half, float (&val)[KL], uint32_t (&idx)[KL])
+      __attribute__((always_inline)) {
+    float v[NR];
+    double x[NR];
+    if constexpr (FULL) {
+#pragma unroll
+      for (int e = 0; e < NR; e += 4) {
+        const float4 q = *reinterpret_cast<const float4*>(half + e);
+        v[e] = q.x;
+        v[e + 1] = q.y;
+        v[e + 2] = q.z;
+        v[e + 3] = q.w;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < NR; ++e) v[e] = half[e < root ? e : 0];
+    }
+#pragma unroll
+    for (int e = 0; e < NR; ++e) {
+      // -0.0 + 0.0 is +0.0: equal scores get equal keys
+      x[e] = route_pack(v[e] + 0.0f, static_cast<uint32_t>(NR - 1 - e));
+      if (!FULL && e >= root) x[e] = kRouteAbsent;
+    }
+    network_top<NR, KL>(x);
+#pragma unroll
+    for (int i = 0; i < KL; ++i) {
+      val[i] = route_score(x[i]);
+      idx[i] = NR - 1 - route_code(x[i]);
+    }
+  };
+  shortlist(projected, fv, fi);
+  shortlist(projected + root, sv, si);
+#pragma unroll
+  for (int i = 0; i < KL; ++i) fi[i] *= static_cast<uint32_t>(root);   // its first slot
+
+  // 2. the pairs with (a+1)(b+1) <= KP hold the KP best (see
+  // product_key_route_row).  Along a row or a column of them the keys
+  // descend, so they are merged as sorted lists, row r from (r, r) on and
+  // column r from (r + 1, r) on; what lies at r >= 2 is sorted at once.  A
+  // key's code: its position, first a, then b, inverted; below it the slot.
+  // A sum of two of these scores is never -0.0.
+  auto pair = [&](int a, int b) __attribute__((always_inline)) {
+    const uint32_t code = (static_cast<uint32_t>(KL * KL - 1 - (a * KL + b)) << 12) |
+                          (fi[a] + si[b]);
+    const double key = route_pack(fv[a] + sv[b], code);
+    return FULL || (a < sub && b < sub) ? key : kRouteAbsent;
+  };
+  double top[KP];
+#pragma unroll
+  for (int b = 0; b < KP; ++b) top[b] = b < KL ? pair(0, b) : kRouteAbsent;
+  auto merge_line = [&](auto row, auto by_row) __attribute__((always_inline)) {
+    constexpr int r = decltype(row)::value;
+    constexpr bool R = decltype(by_row)::value;
+    constexpr int first = R ? r : r + 1;
+    constexpr int end = KP / (r + 1) < KL ? KP / (r + 1) : KL;
+    if constexpr (end > first) {
+      double list[end - first];
+#pragma unroll
+      for (int i = first; i < end; ++i) list[i - first] = R ? pair(r, i) : pair(i, r);
+      merge_top<KP, end - first>(top, list);
+    }
+  };
+  using std::integral_constant;
+  merge_line(integral_constant<int, 0>{}, std::false_type{});
+  merge_line(integral_constant<int, 1>{}, std::true_type{});
+  merge_line(integral_constant<int, 1>{}, std::false_type{});
+  constexpr int tail = [] {
+    int n = 0;
+    for (int a = 2; a < KL; ++a) {
+      for (int b = 2; b < KL; ++b) n += (a + 1) * (b + 1) <= KP ? 1 : 0;
+    }
+    return n;
+  }();
+  if constexpr (tail > 0) {
+    constexpr int TP = route_pow2(tail);
+    double rest[TP];
+#pragma unroll
+    for (int i = tail; i < TP; ++i) rest[i] = kRouteAbsent;
+    int n = 0;
+#pragma unroll
+    for (int a = 2; a < KL; ++a) {
+#pragma unroll
+      for (int b = 2; b < KL; ++b) {
+        if ((a + 1) * (b + 1) <= KP) rest[n++] = pair(a, b);
+      }
+    }
+    network_sort<TP>(rest);
+    merge_top<KP, TP>(top, rest);
+  }
+
+  // 3. softmax of the final_k best, summed in product_key_route_row's order
+  // (lane i there with lanes i ^ 16, i ^ 8, ...), then sorted by slot
+  const float mx = route_score(top[0]);
+  constexpr int EP = KP < 2 ? 2 : KP;
+  float e[EP], part[EP];
+#pragma unroll
+  for (int i = 0; i < KP; ++i) {
+    e[i] = FULL || i < final_k ? expf(route_score(top[i]) - mx) : 0.0f;
+    part[i] = e[i];
+  }
+#pragma unroll
+  for (int d = KP / 2; d > 0; d /= 2) {
+#pragma unroll
+    for (int i = 0; i < d; ++i) part[i] = part[i] + part[i + d];
+  }
+  const float total = part[0];
+#pragma unroll
+  for (int i = 0; i < KP; ++i) {
+    // ascending slots from the highest key down, routes past final_k last
+    const uint32_t slot = route_code(top[i]) & 0xfffu;
+    top[i] = __hiloint2double(
+        static_cast<int>(0x20000fffu - (FULL || i < final_k ? slot : 0x1000u)),
+        __float_as_int(e[i] / total));
+  }
+  network_sort<KP>(top);
+  if (on) {
+#pragma unroll
+    for (int i = 0; i < KP; ++i) {
+      if (FULL || i < final_k) {
+        weights[i] = __int_as_float(__double2loint(top[i]));
+        indices[i] = 0x20000fffu - static_cast<uint32_t>(__double2hiint(top[i]));
+      }
+    }
+  }
+}
+
+constexpr int kRouteLaneRoot = 32;
+constexpr int kRouteLaneRows = 4096;   // see cowsdm_product_key_routes
 
 // The selection's shape for N slots and `selected` routes a row: root =
 // sqrt(N), sub = min(selected, root) entries shortlisted per half, final_k =

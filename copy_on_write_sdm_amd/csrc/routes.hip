@@ -1,5 +1,5 @@
-// cowsdm_product_key_routes: one wave per route row (routes.h holds the
-// selection), kRouteWaves rows per workgroup.
+// cowsdm_product_key_routes: one lane or one wave per route row (routes.h
+// holds both selections, which give the same bits).
 
 #include "routes.h"
 
@@ -18,6 +18,51 @@ __global__ __launch_bounds__(kWave * kRouteWaves) void product_key_routes_kernel
   if (row >= rows) return;
   product_key_route_row<J, M>(projected, row, root, sub, final_k, weights, indices,
                               stage_val[wave], stage_pos[wave], pool_val[wave], pool_pos[wave]);
+}
+
+// One wave per workgroup, so that few rows still spread over the compute units.
+template <int NR, int KP, bool FULL>
+__global__ __launch_bounds__(kWave) void product_key_routes_lane_kernel(
+    const float* __restrict__ projected, int64_t rows, int root, int sub, int final_k,
+    float* __restrict__ weights, int64_t* __restrict__ indices) {
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * kWave + threadIdx.x;
+  const bool on = row < rows;
+  product_key_route_lane<NR, KP, FULL>(on, projected + (on ? row : 0) * 2 * root, root, sub,
+                                       final_k, weights + row * final_k,
+                                       indices + row * final_k);
+}
+
+// One lane per row, or false where one wave per row is the better one: above
+// sqrt(N) = 32 a row's scores do not fit in a lane's registers, and below
+// kRouteLaneRows rows neither fills the device, so the shorter program wins.
+// That is the lane's where sqrt(N), the shortlist and K fill its networks
+// (64 rows: N = 256 K = 16 5.7 us against 6.2, K = 4 3.7 against 4.4, N =
+// 1,024 K = 32 11.9 against 12.1) and the wave's otherwise (N = 64 K = 16
+// 5.3 us against 7.5, N = 400 K = 8 5.2 against 5.7, N = 1,024 K = 24 11.1
+// against 15.2).  At 4,096 rows the lane is ahead or even for all of these
+// (6.0 us against 9.6, 8.0 against 8.0, 15.9 against 20.2).
+template <int NR, int KP>
+bool launch_routes_lane_k(const float* projected, int64_t rows, int root, int sub, int final_k,
+                          float* weights, int64_t* indices, hipStream_t stream) {
+  const bool full = root == NR && sub == (KP < NR ? KP : NR) && final_k == KP &&
+                    reinterpret_cast<uintptr_t>(projected) % 16 == 0;
+  if (!full && rows < kRouteLaneRows) return false;
+  auto* const kernel = full ? &product_key_routes_lane_kernel<NR, KP, true>
+                            : &product_key_routes_lane_kernel<NR, KP, false>;
+  const int64_t blocks = (rows + kWave - 1) / kWave;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kWave), 0, stream,
+                     projected, rows, root, sub, final_k, weights, indices);
+  return true;
+}
+
+template <int NR>
+bool launch_routes_lane(const float* projected, int64_t rows, int root, int sub, int final_k,
+                        float* weights, int64_t* indices, hipStream_t stream) {
+  auto* const launch = final_k <= 4    ? &launch_routes_lane_k<NR, 4>
+                       : final_k <= 8  ? &launch_routes_lane_k<NR, 8>
+                       : final_k <= 16 ? &launch_routes_lane_k<NR, 16>
+                                       : &launch_routes_lane_k<NR, 32>;
+  return launch(projected, rows, root, sub, final_k, weights, indices, stream);
 }
 
 template <int J, int M>
@@ -57,6 +102,12 @@ extern "C" int32_t cowsdm_product_key_routes(const float* projected, int64_t row
   if (!projected || !weights || !indices)
     return fail(-1, "product_key_routes: null pointer argument");
   auto s = static_cast<hipStream_t>(stream);
+  const bool lane =
+      r <= 16 ? launch_routes_lane<16>(projected, rows, r, k, f, weights, indices, s)
+      : r <= kRouteLaneRoot
+          ? launch_routes_lane<kRouteLaneRoot>(projected, rows, r, k, f, weights, indices, s)
+          : false;
+  if (lane) return launch_status("product_key_routes");
   if (r <= kWave)
     launch_routes_pairs<1>(projected, rows, r, k, f, weights, indices, s);
   else if (r <= 4 * kWave)
