@@ -446,22 +446,38 @@ struct RouteStage {
   int pool_pos[kCtlMaxWaves][kWave];
 };
 
+// M: how a row's routes are selected, 0 sorted across lanes (then the stage
+// is not used), else product_key_route_row's M
+template <int M>
+__device__ __forceinline__ void controller_route_row(const float* keys, int64_t row, int root,
+                                                     int sub, int k, float* weights,
+                                                     int64_t* indices, RouteStage* st,
+                                                     int wave) {
+  if constexpr (M == 0) {
+    product_key_route_row_sorted(keys, row, root, sub, k, weights, indices);
+  } else {
+    product_key_route_row<1, M>(keys, row, root, sub, k, weights, indices, st->val[wave],
+                                st->pos[wave], st->pool_val[wave], st->pool_pos[wave]);
+  }
+}
+
 template <int MR, int MW>
-__device__ __forceinline__ void controller_routes_part(const CtlParams& P, const CtlRoutes& R,
-                                                       RouteStage& st) {
+__device__ __forceinline__ void controller_routes_part(const CtlParams& P, const CtlRoutes& R) {
+  RouteStage* stage = nullptr;
+  if constexpr (MR + MW > 0) {
+    __shared__ RouteStage shared;
+    stage = &shared;
+  }
   const int64_t b0 = static_cast<int64_t>(blockIdx.x) * P.tokens_per_group;
   const int rows = group_tokens(P, b0) * P.heads;
   const int wave = static_cast<int>(threadIdx.x) / kWave;
   for (int task = wave; task < 2 * rows; task += static_cast<int>(blockDim.x) / kWave) {
     if (task < rows) {
-      product_key_route_row<1, MR>(P.read_keys, b0 * P.heads + task, R.root, R.read_sub,
-                                   R.read_k, R.read_weights, R.read_indices, st.val[wave],
-                                   st.pos[wave], st.pool_val[wave], st.pool_pos[wave]);
+      controller_route_row<MR>(P.read_keys, b0 * P.heads + task, R.root, R.read_sub, R.read_k,
+                               R.read_weights, R.read_indices, stage, wave);
     } else {
-      product_key_route_row<1, MW>(P.write_keys, b0 * P.heads + task - rows, R.root,
-                                   R.write_sub, R.write_k, R.write_weights, R.write_indices,
-                                   st.val[wave], st.pos[wave], st.pool_val[wave],
-                                   st.pool_pos[wave]);
+      controller_route_row<MW>(P.write_keys, b0 * P.heads + task - rows, R.root, R.write_sub,
+                               R.write_k, R.write_weights, R.write_indices, stage, wave);
     }
   }
 }
@@ -471,7 +487,6 @@ template <int MR, int MW>
 __global__ __launch_bounds__(kCtlThreads) void controller_prepare_routes_kernel(CtlParams P,
                                                                                 CtlRoutes R) {
   extern __shared__ float lds[];
-  __shared__ RouteStage stage;
   const int tiles = (P.rows + kCtlTile - 1) / kCtlTile;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
   CtlWeights<1, ctl_chunk<1, 1>()> weights;
@@ -480,7 +495,7 @@ __global__ __launch_bounds__(kCtlThreads) void controller_prepare_routes_kernel(
   }
   controller_prepare_body<1, 1, false>(P, lds, weights, 0, tiles, true);
   __syncthreads();
-  controller_routes_part<MR, MW>(P, R, stage);
+  controller_routes_part<MR, MW>(P, R);
 }
 
 // finish of the workgroup's tokens.  lds: the normalised inputs, then the
@@ -605,7 +620,6 @@ template <int MR, int MW>
 __global__ __launch_bounds__(kCtlThreads) void controller_finish_prepare_routes_kernel(
     CtlParams F, CtlParams P, CtlRoutes R, int split) {
   extern __shared__ float lds[];
-  __shared__ RouteStage stage;
   const int tiles = (P.rows + kCtlTile - 1) / kCtlTile;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
   CtlWeights<1, ctl_chunk<1, 1>()> finish, weights;
@@ -617,7 +631,7 @@ __global__ __launch_bounds__(kCtlThreads) void controller_finish_prepare_routes_
   __syncthreads();
   controller_prepare_body<1, 1, true>(P, lds, weights, 0, tiles, true);
   __syncthreads();
-  controller_routes_part<MR, MW>(P, R, stage);
+  controller_routes_part<MR, MW>(P, R);
 }
 
 namespace {
@@ -797,6 +811,11 @@ int32_t by_tokens(const CtlParams& P, int lds_rows, One one, Two two, Many many)
   return even && P.batch > kCtlFewTokens ? two() : one();
 }
 
+// How a wave selects its rows' routes (controller_route_row's M).
+int route_m(const CtlRoutes& R, int sub, int k) {
+  return route_row_sorted(R.root, k) ? 0 : route_pair_m(sub, k);
+}
+
 // The route geometry of `reads` and `writes` selections over c's slots and
 // the four output pointers (checked once batch > 0).
 int32_t route_params(const cowsdm_controller_t* c, int64_t batch, int64_t reads, int64_t writes,
@@ -891,11 +910,12 @@ extern "C" int32_t cowsdm_controller_prepare_routes(
     return cowsdm_product_key_routes(write_keys, rows, c->slots, writes, write_weights,
                                      write_indices, stream);
   }
-  const int mr = route_pair_m(R.read_sub, R.read_k), mw = route_pair_m(R.write_sub, R.write_k);
-  if (mr == 1 && mw == 1) return launch_prepare_routes<1, 1>(P, R, s);
-  if (mr == 1) return launch_prepare_routes<1, 2>(P, R, s);
-  if (mw == 1) return launch_prepare_routes<2, 1>(P, R, s);
-  return launch_prepare_routes<2, 2>(P, R, s);
+  const int mr = route_m(R, R.read_sub, R.read_k), mw = route_m(R, R.write_sub, R.write_k);
+  if (mr == 0 && mw == 0) return launch_prepare_routes<0, 0>(P, R, s);
+  if (mr == 0) return mw == 1 ? launch_prepare_routes<0, 1>(P, R, s) : launch_prepare_routes<0, 2>(P, R, s);
+  if (mw == 0) return mr == 1 ? launch_prepare_routes<1, 0>(P, R, s) : launch_prepare_routes<2, 0>(P, R, s);
+  if (mr == 1) return mw == 1 ? launch_prepare_routes<1, 1>(P, R, s) : launch_prepare_routes<1, 2>(P, R, s);
+  return mw == 1 ? launch_prepare_routes<2, 1>(P, R, s) : launch_prepare_routes<2, 2>(P, R, s);
 }
 
 extern "C" int32_t cowsdm_controller_finish_residual(const cowsdm_controller_t* c,
@@ -961,9 +981,10 @@ extern "C" int32_t cowsdm_controller_finish_prepare_routes(
                                             write_weights, write_indices, stream);
   }
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  const int mr = route_pair_m(R.read_sub, R.read_k), mw = route_pair_m(R.write_sub, R.write_k);
-  if (mr == 1 && mw == 1) return launch_finish_prepare_routes<1, 1>(F, P, R, s);
-  if (mr == 1) return launch_finish_prepare_routes<1, 2>(F, P, R, s);
-  if (mw == 1) return launch_finish_prepare_routes<2, 1>(F, P, R, s);
-  return launch_finish_prepare_routes<2, 2>(F, P, R, s);
+  const int mr = route_m(R, R.read_sub, R.read_k), mw = route_m(R, R.write_sub, R.write_k);
+  if (mr == 0 && mw == 0) return launch_finish_prepare_routes<0, 0>(F, P, R, s);
+  if (mr == 0) return mw == 1 ? launch_finish_prepare_routes<0, 1>(F, P, R, s) : launch_finish_prepare_routes<0, 2>(F, P, R, s);
+  if (mw == 0) return mr == 1 ? launch_finish_prepare_routes<1, 0>(F, P, R, s) : launch_finish_prepare_routes<2, 0>(F, P, R, s);
+  if (mr == 1) return mw == 1 ? launch_finish_prepare_routes<1, 1>(F, P, R, s) : launch_finish_prepare_routes<1, 2>(F, P, R, s);
+  return mw == 1 ? launch_finish_prepare_routes<2, 1>(F, P, R, s) : launch_finish_prepare_routes<2, 2>(F, P, R, s);
 }

@@ -517,6 +517,162 @@ __device__ __forceinline__ void product_key_route_lane(bool on,
 constexpr int kRouteLaneRoot = 32;
 constexpr int kRouteLaneRows = 4096;   // see cowsdm_product_key_routes
 
+// ---- One wave per row, few routes (sqrt(N) <= 32, K <= 16) ------------------
+//
+// product_key_route_row for a decode step's few rows, where the latency of
+// one row is what counts: the same keys and the same pairs as the lane form,
+// sorted across lanes.  A step of a bitonic sort is a DPP move of the key and
+// a v_max_f64 / v_min_f64 (only the three moves between rows of 16 lanes go
+// through ds_bpermute), so the selection is about 400 instructions without
+// LDS staging, against about 900 and a dozen waits on LDS.
+// 64 rows, launch included: N = 256 K = 16 6.2 -> 3.5 us, K = 4 4.4 -> 3.4,
+// N = 1,024 K = 16 6.3 -> 3.3, N = 400 K = 8 5.2 -> 3.4.
+
+// The key of lane ^ 1, ^ 2, ^ 4, ^ 8 (STEP 1, 2, 4, 8) or of the mirrored lane
+// of 4, 8 or 16 (STEP 3, 7, 15).
+template <int STEP>
+__device__ __forceinline__ int lane_partner(int x) {
+  if constexpr (STEP == 4) {
+    // lanes 0-3 and 8-11 of a row from four above, the others from four below
+    const int up = __builtin_amdgcn_update_dpp(0, x, 0x104, 0xf, 0x5, true);
+    return __builtin_amdgcn_update_dpp(up, x, 0x114, 0xf, 0xa, false);
+  } else {
+    constexpr int ctrl = STEP == 1    ? 0xB1    // quad_perm [1,0,3,2]
+                         : STEP == 2  ? 0x4E    // quad_perm [2,3,0,1]
+                         : STEP == 3  ? 0x1B    // quad_perm [3,2,1,0]
+                         : STEP == 7  ? 0x141   // row_half_mirror
+                         : STEP == 8  ? 0x128   // row_ror:8
+                                      : 0x140;  // row_mirror
+    return __builtin_amdgcn_update_dpp(0, x, ctrl, 0xf, 0xf, true);
+  }
+}
+
+// One step of a descending sort within rows of 16 lanes: the lane whose
+// highest bit of STEP is 0 keeps the higher key.
+template <int STEP>
+__device__ __forceinline__ double row_step(double key, int lane) {
+  constexpr int bit = STEP == 3 ? 2 : STEP == 7 ? 4 : STEP == 15 ? 8 : STEP;
+  const double other = __hiloint2double(lane_partner<STEP>(__double2hiint(key)),
+                                        lane_partner<STEP>(__double2loint(key)));
+  const double high = key_max(key, other), low = key_min(key, other);
+  return (lane & bit) == 0 ? high : low;
+}
+
+// a bitonic row into descending order
+__device__ __forceinline__ double row_clean(double key, int lane) {
+  key = row_step<8>(key, lane);
+  key = row_step<4>(key, lane);
+  key = row_step<2>(key, lane);
+  return row_step<1>(key, lane);
+}
+
+__device__ __forceinline__ double row_sort(double key, int lane) {
+  key = row_step<1>(key, lane);
+  key = row_step<3>(key, lane);
+  key = row_step<1>(key, lane);
+  key = row_step<7>(key, lane);
+  key = row_step<2>(key, lane);
+  key = row_step<1>(key, lane);
+  key = row_step<15>(key, lane);
+  key = row_step<4>(key, lane);
+  key = row_step<2>(key, lane);
+  return row_step<1>(key, lane);
+}
+
+__device__ __forceinline__ double lane_key(double key, int lane) {
+  return __hiloint2double(__builtin_amdgcn_ds_bpermute(4 * lane, __double2hiint(key)),
+                          __builtin_amdgcn_ds_bpermute(4 * lane, __double2loint(key)));
+}
+
+// Two descending rows, `flip` ^ lane apart (31 or 63: the mirrored lanes of
+// neighbouring rows or pairs of rows), into the 16 highest of both,
+// descending, in either.
+__device__ __forceinline__ double row_merge(double key, int lane, int flip) {
+  return row_clean(key_max(key, lane_key(key, lane ^ flip)), lane);
+}
+
+// Row `row` of `projected` by the calling wave; root <= 32, final_k <= 16.
+__device__ __forceinline__ void product_key_route_row_sorted(
+    const float* __restrict__ projected, int64_t row, int root, int sub, int final_k,
+    float* __restrict__ weights, int64_t* __restrict__ indices) {
+  const int lane = static_cast<int>(threadIdx.x) % kWave;
+  const float* const first = projected + row * 2 * root;
+  // 1. the halves' shortlists: sqrt(N) <= 16 the first half in the lanes of
+  // row 0 and the second in those of row 1, above that two rows each
+  const bool wide = root > 16;
+  const int per = wide ? 32 : 16;          // lanes of a half
+  const int e = lane % per, half = lane / per;
+  const bool in = half < 2 && e < root;
+  const float v = first[in ? half * root + e : 0];
+  double key = in ? route_pack(v + 0.0f, static_cast<uint32_t>(31 - e)) : kRouteAbsent;
+  key = row_sort(key, lane);
+  if (wide) key = row_merge(key, lane, 31);
+
+  // 2. the pairs with (a+1)(b+1) <= 16, a row or a column of them to a row
+  // of lanes where it fills one: (0, b); (a, 0); (1, b) and (a, 1); the rest
+  const int i = lane % 16;
+  int a = 0, b = i;
+  if (lane >= 48) {
+    a = i < 3 ? 2 : i == 4 ? 4 : 3;        // (2,2) (2,3) (2,4) (3,2) (4,2) (3,3)
+    b = i < 3 ? i + 2 : i == 5 ? 3 : 2;
+    if (i > 5) b = 16;
+  } else if (lane >= 32) {
+    a = i < 7 ? 1 : i - 5;                 // (1,1) .. (1,7), (2,1) .. (7,1)
+    b = i < 7 ? i + 1 : 1;
+    if (i > 12) b = 16;
+  } else if (lane >= 16) {
+    a = i + 1;                             // (1,0) .. (15,0)
+    b = 0;
+  }
+  const double fk = lane_key(key, a % 16), sk = lane_key(key, per + b % 16);
+  const uint32_t slot = (31 - route_code(fk)) * static_cast<uint32_t>(root) +
+                        (31 - route_code(sk));
+  const uint32_t code = (static_cast<uint32_t>(255 - (a * 16 + b)) << 12) | slot;
+  double top = a < sub && b < sub ? route_pack(route_score(fk) + route_score(sk), code)
+                                  : kRouteAbsent;
+  top = row_merge(row_merge(row_sort(top, lane), lane, 31), lane, 63);
+
+  // 3. every row of lanes holds the 16 best: softmax of the first final_k,
+  // summed in product_key_route_row's order, then each one's place by slot
+  const float score = route_score(top);
+  const float mx = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(score)));
+  const bool mine = i < final_k;
+  const float ex = mine ? expf(score - mx) : 0.0f;
+  float total = ex;
+  total += __int_as_float(lane_partner<8>(__float_as_int(total)));
+  total += __int_as_float(lane_partner<4>(__float_as_int(total)));
+  total += __int_as_float(lane_partner<2>(__float_as_int(total)));
+  total += __int_as_float(lane_partner<1>(__float_as_int(total)));
+  const int own = mine ? static_cast<int>(route_code(top) & 0xfffu) : 0x1000 + i;
+  int rank = 0;
+#define COWSDM_ROUTE_RANK(r) \
+  rank += __builtin_amdgcn_update_dpp(0, own, 0x120 + r, 0xf, 0xf, true) < own ? 1 : 0
+  COWSDM_ROUTE_RANK(1);
+  COWSDM_ROUTE_RANK(2);
+  COWSDM_ROUTE_RANK(3);
+  COWSDM_ROUTE_RANK(4);
+  COWSDM_ROUTE_RANK(5);
+  COWSDM_ROUTE_RANK(6);
+  COWSDM_ROUTE_RANK(7);
+  COWSDM_ROUTE_RANK(8);
+  COWSDM_ROUTE_RANK(9);
+  COWSDM_ROUTE_RANK(10);
+  COWSDM_ROUTE_RANK(11);
+  COWSDM_ROUTE_RANK(12);
+  COWSDM_ROUTE_RANK(13);
+  COWSDM_ROUTE_RANK(14);
+  COWSDM_ROUTE_RANK(15);
+#undef COWSDM_ROUTE_RANK
+  if (lane < 16 && mine) {
+    weights[row * final_k + rank] = ex / total;
+    indices[row * final_k + rank] = own;
+  }
+}
+
+// Whether a row's routes are selected by product_key_route_row_sorted when a
+// wave has the row (the pairs' rows of lanes hold 16 of a shortlist).
+inline bool route_row_sorted(int root, int final_k) { return root <= 32 && final_k <= 16; }
+
 // The selection's shape for N slots and `selected` routes a row: root =
 // sqrt(N), sub = min(selected, root) entries shortlisted per half, final_k =
 // min(selected, sub * sub) routes; 0, or the error of

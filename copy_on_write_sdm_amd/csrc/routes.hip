@@ -1,5 +1,5 @@
 // cowsdm_product_key_routes: one lane or one wave per route row (routes.h
-// holds both selections, which give the same bits).
+// holds the selections, which give the same bits).
 
 #include "routes.h"
 
@@ -32,21 +32,24 @@ __global__ __launch_bounds__(kWave) void product_key_routes_lane_kernel(
                                        indices + row * final_k);
 }
 
-// One lane per row, or false where one wave per row is the better one: above
-// sqrt(N) = 32 a row's scores do not fit in a lane's registers, and below
-// kRouteLaneRows rows neither fills the device, so the shorter program wins.
-// That is the lane's where sqrt(N), the shortlist and K fill its networks
-// (64 rows: N = 256 K = 16 5.7 us against 6.2, K = 4 3.7 against 4.4, N =
-// 1,024 K = 32 11.9 against 12.1) and the wave's otherwise (N = 64 K = 16
-// 5.3 us against 7.5, N = 400 K = 8 5.2 against 5.7, N = 1,024 K = 24 11.1
-// against 15.2).  At 4,096 rows the lane is ahead or even for all of these
-// (6.0 us against 9.6, 8.0 against 8.0, 15.9 against 20.2).
+// One lane per row, or false where one wave per row is the better one.  Above
+// sqrt(N) = 32 a row's scores do not fit in a lane's registers.  Below a few
+// thousand rows neither fills the device and the shorter program wins: the
+// sorted wave's where it applies (N = 256 K = 16: 3.4 us to 2,048 rows and
+// 4.4 at 4,000, the lane's 5.7 to 6.3 at 8,192; K = 4: 3.4 to 4.5 against
+// 3.6); for more routes the lane's if sqrt(N), the shortlist and K fill its
+// networks (N = 1,024 K = 32, 64 rows: 11.9 us against 12.1) and the ranking
+// wave's otherwise (N = 1,024 K = 24, 64 rows: 11.1 us against 15.2; 4,096
+// rows: 20.2 against 15.9).
 template <int NR, int KP>
 bool launch_routes_lane_k(const float* projected, int64_t rows, int root, int sub, int final_k,
                           float* weights, int64_t* indices, hipStream_t stream) {
   const bool full = root == NR && sub == (KP < NR ? KP : NR) && final_k == KP &&
                     reinterpret_cast<uintptr_t>(projected) % 16 == 0;
-  if (!full && rows < kRouteLaneRows) return false;
+  const bool sorted = route_row_sorted(root, final_k);
+  if (sorted ? rows < kRouteLaneRows * (final_k > 8 ? 2 : 1) : !full && rows < kRouteLaneRows) {
+    return false;
+  }
   auto* const kernel = full ? &product_key_routes_lane_kernel<NR, KP, true>
                             : &product_key_routes_lane_kernel<NR, KP, false>;
   const int64_t blocks = (rows + kWave - 1) / kWave;
@@ -63,6 +66,15 @@ bool launch_routes_lane(const float* projected, int64_t rows, int root, int sub,
                        : final_k <= 16 ? &launch_routes_lane_k<NR, 16>
                                        : &launch_routes_lane_k<NR, 32>;
   return launch(projected, rows, root, sub, final_k, weights, indices, stream);
+}
+
+__global__ __launch_bounds__(kWave * kRouteWaves) void product_key_routes_sorted_kernel(
+    const float* __restrict__ projected, int64_t rows, int root, int sub, int final_k,
+    float* __restrict__ weights, int64_t* __restrict__ indices) {
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * kRouteWaves +
+                      static_cast<int>(threadIdx.x) / kWave;
+  if (row >= rows) return;
+  product_key_route_row_sorted(projected, row, root, sub, final_k, weights, indices);
 }
 
 template <int J, int M>
@@ -108,7 +120,12 @@ extern "C" int32_t cowsdm_product_key_routes(const float* projected, int64_t row
           ? launch_routes_lane<kRouteLaneRoot>(projected, rows, r, k, f, weights, indices, s)
           : false;
   if (lane) return launch_status("product_key_routes");
-  if (r <= kWave)
+  if (route_row_sorted(r, f)) {
+    hipLaunchKernelGGL(product_key_routes_sorted_kernel,
+                       dim3(static_cast<uint32_t>((rows + kRouteWaves - 1) / kRouteWaves)),
+                       dim3(kWave * kRouteWaves), 0, s, projected, rows, r, k, f, weights,
+                       indices);
+  } else if (r <= kWave)
     launch_routes_pairs<1>(projected, rows, r, k, f, weights, indices, s);
   else if (r <= 4 * kWave)
     launch_routes_pairs<4>(projected, rows, r, k, f, weights, indices, s);
