@@ -684,7 +684,6 @@ class PackedSDMCopyOnWriteState:
         self.slab_buffers = (vbuf, fbuf)
         self.values, self.free_rows = vbuf[:capacity], fbuf[:capacity]
 
-    @torch.no_grad()
     def prepare_step_capacity(self, maximum_new_rows: int) -> int:
         """Prove one fused decode step, growing pooled headroom if short
         (allocator.py:745-773).  Host bookkeeping; reads free_count only
@@ -756,13 +755,13 @@ class PackedSDMCopyOnWriteState:
         return capacities
 
     def _read_free_count(self) -> int:
-        """free_count, read with the kernels' sticky error word (one
-        transfer); raises when a step stopped on a fault."""
+        """free_count, read with the kernels' sticky error word; raises when
+        a step stopped on a fault.  Two reads: the second finds the stream
+        idle, and both together cost less than gathering the words first."""
 
-        words = torch.stack([self.free_count.to(torch.int64),
-                             self.ensure_scratch()[nat.SCRATCH_ERRORS]]).tolist()
-        self._raise_on_fault(words[1])
-        return int(words[0])
+        free_rows = int(self.free_count.item())
+        self._raise_on_fault(int(self.ensure_scratch()[nat.SCRATCH_ERRORS].item()))
+        return free_rows
 
     @staticmethod
     def _raise_on_fault(errors: int) -> None:
@@ -1120,8 +1119,9 @@ class PackedSDMCopyOnWriteState:
         }
 
     def ensure_scratch(self) -> torch.Tensor:
-        if self.scratch is None or self.scratch.numel() != int(
-                nat.lib().cowsdm_step_scratch_words(self.banks)):
+        # cowsdm_step_scratch_words: one look-back slot per bank after the
+        # fixed words
+        if self.scratch is None or self.scratch.numel() != nat.SCRATCH_SLOTS + self.banks:
             self.scratch = _scratch(self.banks, self.values.device)
         return self.scratch
 
@@ -1243,40 +1243,25 @@ def _step_layer(
     write_indices, write_weights, values, input_gate, erase_gate, forget_log_gate,
     read_indices, read_weights, output, first, repeated, allocated,
 ) -> nat.Layer:
-    layer = nat.Layer()
-    if state is not None:
-        layer.shared_initial_memory = state.shared_initial_memory.data_ptr()
-        layer.template_indices = state.template_indices.data_ptr()
-        layer.values = state.values.data_ptr()
-        paged = state.paged_map
-        if paged is None:
-            layer.logical_to_physical = state.logical_to_physical.data_ptr()
-        else:
-            layer.map_directory = paged.directory.data_ptr()
-            layer.map_pages = paged.pages.data_ptr()
-            layer.map_page_count = paged.page_count.data_ptr()
-            layer.map_page_capacity = paged.capacity
-            layer.map_page_shift = paged.page_shift
-        layer.free_rows = state.free_rows.data_ptr()
-        layer.free_count = state.free_count.data_ptr()
-        layer.overflow_flag = state.overflow_flag.data_ptr()
-        layer.scratch = state.ensure_scratch().data_ptr()
-        layer.capacity_rows = state.capacity_rows
-    else:
-        layer.values = memory.data_ptr()
-        layer.capacity_rows = 0
-    layer.write_indices = write_indices.data_ptr()
-    layer.write_weights = write_weights.data_ptr()
-    layer.step_values = values.data_ptr()
-    layer.input_gate = input_gate.data_ptr()
-    layer.erase_gate = erase_gate.data_ptr()
-    layer.forget_log_gate = forget_log_gate.data_ptr()
-    layer.read_indices = read_indices.data_ptr()
-    layer.read_weights = read_weights.data_ptr()
-    layer.output = output.data_ptr()
-    layer.first_touches_out = nat.ptr(first)
-    layer.repeated_writes_out = nat.ptr(repeated)
-    layer.allocated_rows_out = nat.ptr(allocated)
+    inputs = (write_indices.data_ptr(), write_weights.data_ptr(), values.data_ptr(),
+              input_gate.data_ptr(), erase_gate.data_ptr(), forget_log_gate.data_ptr(),
+              read_indices.data_ptr(), read_weights.data_ptr(), output.data_ptr(),
+              nat.ptr(first), nat.ptr(repeated), nat.ptr(allocated))
+    if state is None:
+        return nat.Layer(None, None, memory.data_ptr(), None, None, None, None, None, 0, *inputs)
+    paged = state.paged_map
+    layer = nat.Layer(
+        state.shared_initial_memory.data_ptr(), state.template_indices.data_ptr(),
+        state.values.data_ptr(),
+        state.logical_to_physical.data_ptr() if paged is None else None,
+        state.free_rows.data_ptr(), state.free_count.data_ptr(), state.overflow_flag.data_ptr(),
+        state.ensure_scratch().data_ptr(), state.capacity_rows, *inputs)
+    if paged is not None:
+        layer.map_directory = paged.directory.data_ptr()
+        layer.map_pages = paged.pages.data_ptr()
+        layer.map_page_count = paged.page_count.data_ptr()
+        layer.map_page_capacity = paged.capacity
+        layer.map_page_shift = paged.page_shift
     return layer
 
 
@@ -1305,18 +1290,9 @@ def _check_step_inputs(banks, slots, width, device, write_indices, write_weights
 
 
 def _shape(banks, slots, width, writes, reads, templates, index_code) -> nat.Shape:
-    shape = nat.Shape()
-    shape.banks = banks
-    shape.slots = slots
-    shape.width = width
-    shape.writes = writes
-    shape.reads = reads
-    shape.templates = templates
-    shape.index_dtype = index_code
-    return shape
+    return nat.Shape(banks, slots, width, writes, reads, templates, index_code)
 
 
-@torch.no_grad()
 def packed_sdm_cow_step(
     state: PackedSDMCopyOnWriteState,
     write_indices: torch.Tensor,

@@ -18,14 +18,13 @@ from __future__ import annotations
 
 import math
 from dataclasses import dataclass, field
-from typing import Any
+from typing import Any, Sequence
 
 import torch
 
 from . import _native as nat
 from .allocator import PackedSDMCopyOnWriteState, dense_sdm_sparse_step, packed_sdm_cow_step
 from .inference import SDMStepInputs
-from .routing import product_key_routes
 
 
 @dataclass
@@ -71,6 +70,14 @@ class SDMController:
     @property
     def device(self) -> torch.device:
         return self.proj_weight_t.device
+
+    def route_counts(self) -> tuple[int, int]:
+        """Read and write routes of a row (product_key_routes, sdm.py:96-159:
+        the shortlists' pairs can be fewer than asked for)."""
+
+        root = math.isqrt(self.slots)
+        return (min(self.reads, min(self.reads, root) ** 2),
+                min(self.writes, min(self.writes, root) ** 2))
 
     # --------------------------------------------------------- creation
 
@@ -231,24 +238,27 @@ def prepare_sdm_step(controller: SDMController, tokens: torch.Tensor) -> Control
     banks = batch * c.memory_heads
     device = tokens.device
     x = tokens.contiguous()
+    reads, writes = c.route_counts()
     normalized = torch.empty(batch, 1, c.width, device=device)
-    read_keys = torch.empty(banks, 1, c.key_width_per_head, device=device)
-    write_keys = torch.empty_like(read_keys)
+    keys = torch.empty(2 * banks * c.key_width_per_head, device=device)
     values = torch.empty(banks, c.head_width, device=device)
-    input_gate = torch.empty(banks, device=device)
-    forget = torch.empty(banks, device=device)
-    nat.check(nat.lib().cowsdm_controller_prepare(
-        c.c_struct(), x.data_ptr(), batch, normalized.data_ptr(), read_keys.data_ptr(),
-        write_keys.data_ptr(), values.data_ptr(), input_gate.data_ptr(), forget.data_ptr(),
-        nat.stream_handle(device)), "cowsdm_controller_prepare")
-    read_weights, read_indices = product_key_routes(read_keys, slots=c.slots, selected=c.reads)
-    write_weights, write_indices = product_key_routes(write_keys, slots=c.slots,
-                                                      selected=c.writes)
+    input_gate, forget = torch.empty(2, banks, device=device)
+    read_weights = torch.empty(banks, reads, device=device)
+    write_weights = torch.empty(banks, writes, device=device)
+    read_indices = torch.empty(banks, reads, device=device, dtype=torch.int64)
+    write_indices = torch.empty(banks, writes, device=device, dtype=torch.int64)
+    read_keys = keys.data_ptr()
+    nat.check(nat.lib().cowsdm_controller_prepare_routes(
+        c.c_struct(), x.data_ptr(), batch, normalized.data_ptr(), read_keys,
+        read_keys + 4 * banks * c.key_width_per_head, values.data_ptr(), input_gate.data_ptr(),
+        forget.data_ptr(), c.reads, c.writes, read_weights.data_ptr(), read_indices.data_ptr(),
+        write_weights.data_ptr(), write_indices.data_ptr(), nat.stream_handle(device)),
+        "cowsdm_controller_prepare_routes")
     return ControllerStep(
         normalized=normalized,
-        inputs=SDMStepInputs(write_indices=write_indices[:, 0], write_weights=write_weights[:, 0],
+        inputs=SDMStepInputs(write_indices=write_indices, write_weights=write_weights,
                              values=values, input_gate=input_gate, forget_log_gate=forget,
-                             read_indices=read_indices[:, 0], read_weights=read_weights[:, 0]))
+                             read_indices=read_indices, read_weights=read_weights))
 
 
 @torch.no_grad()
@@ -291,6 +301,100 @@ def decode_sdm_layer_controller(controller: SDMController, tokens: torch.Tensor,
         x.read_indices, x.read_weights, backend=backend, validate_routes=False,
         collect_diagnostics=False)
     return finish_sdm_step(controller, step, reading)
+
+
+def decode_sdm_layers_controller(controllers: Sequence[SDMController],
+                                 states: Sequence[PackedSDMCopyOnWriteState],
+                                 tokens: torch.Tensor) -> torch.Tensor:
+    """One token through consecutive SDM layers with nothing between them but
+    their residual adds: per layer what ``decode_sdm_layer_controller`` runs,
+    then ``tokens + mixed`` (inference.py:655-660), bit for bit, with a
+    layer's finish, its residual add and the next layer's prepare and routes
+    in one launch.  The layers' states are proven or grow (and prove) here,
+    with direct maps (``can_decode_layers``).  The buffers between the kernels
+    are one allocation of this call, each in two copies that the layers take
+    in turn."""
+
+    batch = tokens.shape[0]
+    for c in controllers:
+        _check_tokens(c, tokens)
+    device = tokens.device
+    lib, stream = nat.lib(), nat.stream_handle(device)
+    layers, size = [], 0
+    for index, c in enumerate(controllers):
+        banks = batch * c.memory_heads
+        reads, writes = c.route_counts()
+        floats = (batch * c.width, banks * c.key_width_per_head, banks * c.key_width_per_head,
+                  batch * c.width, banks, banks, banks * reads, 2 * banks * reads,
+                  banks * writes, 2 * banks * writes, batch * c.width, batch * c.width,
+                  batch * c.width)
+        offsets, at = [], 0
+        for n in floats:
+            offsets.append(at)
+            at += -(-n // 4) * 16        # 16-byte aligned
+        size = max(size, at)
+        layers.append((banks, reads, writes, offsets))
+    work = torch.empty(2 * size, device=device, dtype=torch.uint8)
+    base = work.data_ptr()
+    x = tokens.contiguous()
+    result = torch.empty(batch, 1, controllers[0].width, device=device)
+
+    def buffers(index: int) -> list[int]:
+        return [base + (index % 2) * size + offset for offset in layers[index][3]]
+
+    def prepare(index: int, b: list[int]) -> tuple:
+        return (b[0], b[1], b[2], b[3], b[4], b[5], controllers[index].reads,
+                controllers[index].writes, b[6], b[7], b[8], b[9])
+
+    buf = buffers(0)
+    residual = x.data_ptr()
+    nat.check(lib.cowsdm_controller_prepare_routes(
+        controllers[0].c_struct(), residual, batch, *prepare(0, buf), stream),
+        "cowsdm_controller_prepare_routes")
+    last = len(layers) - 1
+    for index, (c, st) in enumerate(zip(controllers, states)):
+        banks, reads, writes, _ = layers[index]
+        if st.banks != banks:
+            raise ValueError("packed SDM banks do not match batch and memory heads")
+        if st.width != c.head_width:
+            raise ValueError("SDM route weights and values do not align")
+        if st.values.device != device:
+            raise ValueError("SDM COW step tensors must share one device")
+        if st.growth_quantum_rows:
+            st.prepare_step_capacity(banks * c.writes)
+        (_, _, _, values, gate, forget, read_w, read_i, write_w, write_i, reading, out,
+         total) = buf
+        m0 = st.shared_initial_memory
+        layer = nat.Layer(
+            m0.data_ptr(), st.template_indices.data_ptr(), st.values.data_ptr(),
+            st.logical_to_physical.data_ptr(), st.free_rows.data_ptr(),
+            st.free_count.data_ptr(), st.overflow_flag.data_ptr(),
+            st.ensure_scratch().data_ptr(), st.capacity_rows, write_i, write_w, values, gate,
+            gate, forget, read_i, read_w, reading)
+        shape = nat.Shape(banks, st.slots, st.width, writes, reads, m0.shape[0],
+                          nat.INDEX_INT64)
+        nat.check(lib.cowsdm_packed_step(layer, shape, stream), "cowsdm_packed_step")
+        if index == last:
+            nat.check(lib.cowsdm_controller_finish_residual(
+                c.c_struct(), buf[0], reading, batch, out, residual, result.data_ptr(), stream),
+                "cowsdm_controller_finish_residual")
+            return result
+        following = buffers(index + 1)
+        nat.check(lib.cowsdm_controller_finish_prepare_routes(
+            c.c_struct(), buf[0], reading, batch, out, residual, total,
+            controllers[index + 1].c_struct(), *prepare(index + 1, following), stream),
+            "cowsdm_controller_finish_prepare_routes")
+        residual, buf = total, following
+    return result
+
+
+def can_decode_layers(state: PackedSDMCopyOnWriteState, backend: str) -> bool:
+    """Whether ``decode_sdm_layers_controller`` takes a layer's state: a
+    direct map, and a capacity that is proven or that its decode proves (no
+    check of the routes against the slab before the step)."""
+
+    return (backend in ("auto", "hip") and state.paged_map is None and state.banks > 0
+            and (state.growth_quantum_rows > 0 or state.capacity_is_proven))
 
 
 @torch.no_grad()
@@ -363,9 +467,7 @@ class ControllerDecodeGraph:
             banks = batch * c.memory_heads
             if st.banks != banks or st.width != c.head_width or st.slots != c.slots:
                 raise ValueError("packed SDM state does not match batch and controller")
-            root = math.isqrt(c.slots)
-            reads = min(c.reads, min(c.reads, root) ** 2)
-            writes = min(c.writes, min(c.writes, root) ** 2)
+            reads, writes = c.route_counts()
             f32 = dict(device=self.device, dtype=torch.float32)
             i64 = dict(device=self.device, dtype=torch.int64)
             buf = {

@@ -352,7 +352,6 @@ def pack_prefill_layers(
         growth_quantum_rows=growth_quantum_rows)
 
 
-@torch.no_grad()
 def decode_sdm_layer(state: PackedSDMCopyOnWriteState, step: SDMStepInputs, *,
                      backend: str = "auto") -> torch.Tensor:
     """Packed decode of one SDM layer for one token (inference.py:538-566):

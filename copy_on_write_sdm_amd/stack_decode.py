@@ -6,7 +6,8 @@ Every "B" layer runs the device controller step around the packed
 copy-on-write step (``decode_sdm_layer_controller``: controller kernels, the
 two product-key route selections, the capacity proof when the slab grows,
 the fused step, the controller's finish) and adds its output to the
-residual stream.  The model's other parts are the caller's, as in
+residual stream; consecutive ones without a tail between them share launches
+(``decode_sdm_layers_controller``).  The model's other parts are the caller's, as in
 ``prefill_faithful_sdm_stack``:
 
 * ``attention_decode(layer, tokens, key_cache, value_cache, position) ->
@@ -29,7 +30,8 @@ from typing import Callable, Sequence
 
 import torch
 
-from .controller import SDMController, decode_sdm_layer_controller
+from .controller import (SDMController, can_decode_layers, decode_sdm_layer_controller,
+                         decode_sdm_layers_controller)
 from .inference import FaithfulSDMDecodeState
 
 AttentionDecode = Callable[[int, torch.Tensor, torch.Tensor, torch.Tensor, "int | torch.Tensor"],
@@ -119,7 +121,10 @@ def decode_faithful_sdm_stack(
 
     dense_index = 0
     sdm_index = 0
+    done = 0   # layers below this one have run
     for layer, kind in enumerate(layout):
+        if layer < done:
+            continue
         if kind == "A":
             tokens = attention_decode(layer, tokens, state.dense_keys[dense_index],
                                       state.dense_values[dense_index], attention_position)
@@ -127,6 +132,20 @@ def decode_faithful_sdm_stack(
             continue
         if state.sdm_layer_positions[sdm_index] != layer:
             raise ValueError("SDM decode layer ordering is inconsistent")
+        # SDM layers in a row with nothing of the caller's between them run
+        # as one chain of launches
+        run = 0
+        while (sdm_tail is None and layer + run < len(layout) and layout[layer + run] == "B"
+               and state.sdm_layer_positions[sdm_index + run] == layer + run
+               and can_decode_layers(state.sdm_states[sdm_index + run], backend)):
+            run += 1
+        if run:
+            tokens = decode_sdm_layers_controller(
+                controllers[sdm_index:sdm_index + run],
+                state.sdm_states[sdm_index:sdm_index + run], tokens)
+            sdm_index += run
+            done = layer + run
+            continue
         mixed = decode_sdm_layer_controller(controllers[sdm_index], tokens,
                                             state.sdm_states[sdm_index], backend=backend)
         tokens = tokens + mixed
