@@ -32,6 +32,10 @@ BUILD_DIR = PACKAGE_DIR / "_build"
 
 INDEX_INT32 = 0
 INDEX_INT64 = 1
+# cowsdm_packed_step_floats' type codes and its places for them
+FLOAT_TYPES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
+FLOAT_PLACES = (1, 2, 3, 4, 5, 7)
+ELIMIT = -2
 
 ERR_WRITE_INDEX = 0x1
 ERR_READ_INDEX = 0x2
@@ -333,6 +337,10 @@ SIGNATURES: dict[str, tuple] = {
         _I32, [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_double),
                ctypes.POINTER(_I32)]),
     "cowsdm_packed_step": (_I32, [ctypes.POINTER(Layer), ctypes.POINTER(Shape), _P]),
+    "cowsdm_packed_step_floats": (
+        _I32, [ctypes.POINTER(Layer), ctypes.POINTER(Shape), _I32, _P]),
+    "cowsdm_dense_step_floats": (
+        _I32, [ctypes.POINTER(Layer), ctypes.POINTER(Shape), _I32, _P]),
     "cowsdm_packed_step_layers": (
         _I32, [ctypes.POINTER(Layer), _I32, ctypes.POINTER(Shape), _P]),
     "cowsdm_packed_step_trace": (

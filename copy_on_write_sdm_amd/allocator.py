@@ -1180,6 +1180,27 @@ def _widen(tensor: torch.Tensor) -> torch.Tensor:
     return tensor.float() if tensor.dtype in _NARROW_FLOATS else tensor
 
 
+def _narrow_types(tensors: Sequence[torch.Tensor], *, writes: int, reads: int, width: int,
+                  banks: int) -> int:
+    """The float type codes of a step's weights, values and gates (in
+    ``nat.FLOAT_PLACES`` order) when some are 16-bit floats and the step's
+    kernel widens them itself; 0 when all are float32, or when they are
+    widened before it (shapes past that kernel's, strided tensors)."""
+
+    types = 0
+    for tensor, place in zip(tensors, nat.FLOAT_PLACES):
+        if tensor.dtype != torch.float32:
+            code = nat.FLOAT_TYPES.get(tensor.dtype)
+            if code is None or not tensor.is_contiguous():
+                return 0
+            types |= code << (2 * place)
+        elif not tensor.is_contiguous():
+            return 0
+    if types and (writes > 4 or reads > 16 or width > 256 or banks > 256):
+        return 0
+    return types
+
+
 def _check_float_tensors(tensors: Sequence[torch.Tensor]) -> None:
     for tensor in tensors:
         if tensor.dtype != torch.float32:
@@ -1325,33 +1346,45 @@ def packed_sdm_cow_step(
                                    writes=write_indices.shape[1], reads=read_indices.shape[1])
     # float16/bfloat16 weights, values and gates compute in float32; the
     # reading comes back in the values' dtype (allocator.py:1521)
-    reading_dtype = values.dtype
-    write_weights, values, input_gate, effective_erase, forget_log_gate, read_weights = (
-        _widen(t) for t in (write_weights, values, input_gate, effective_erase,
-                            forget_log_gate, read_weights))
-    _check_float_tensors((write_weights, values, input_gate, effective_erase,
-                          forget_log_gate, read_weights))
+    writes, reads = write_indices.shape[1], read_indices.shape[1]
     index_code = _index_code(write_indices, read_indices)
-    output = torch.empty_like(values)
+    types = _narrow_types((write_weights, values, input_gate, effective_erase, forget_log_gate,
+                           read_weights), writes=writes, reads=reads, width=width, banks=banks)
+    reading_dtype = values.dtype
     first = repeated = allocated = None
     if collect_diagnostics:
         first = torch.empty(banks, device=device, dtype=torch.int64)
         repeated = torch.empty(banks, device=device, dtype=torch.int64)
         allocated = torch.empty((), device=device, dtype=torch.int32)
     if state.paged_map is not None and banks:
-        state.paged_map.prove(banks * write_indices.shape[1])
-    layer = _step_layer(state, None, write_indices, write_weights, values, input_gate,
-                        effective_erase, forget_log_gate, read_indices, read_weights, output,
-                        first, repeated, allocated)
-    shape = _shape(banks, slots, width, write_indices.shape[1], read_indices.shape[1],
-                   state.shared_initial_memory.shape[0], index_code)
-    if banks and (validate_routes or torch_checks or not state.capacity_is_proven):
-        _run_precheck(layer, shape, dense=False, unique=validate_routes,
-                      capacity=torch_checks or not state.capacity_is_proven, device=device)
-    if banks:
+        state.paged_map.prove(banks * writes)
+    shape = _shape(banks, slots, width, writes, reads, state.shared_initial_memory.shape[0],
+                   index_code)
+    floats = (write_weights, values, input_gate, effective_erase, forget_log_gate, read_weights)
+    while True:
+        if not types:
+            floats = tuple(_widen(t) for t in floats)
+            _check_float_tensors(floats)
+        write_weights, values, input_gate, effective_erase, forget_log_gate, read_weights = floats
+        output = torch.empty_like(values)
+        layer = _step_layer(state, None, write_indices, write_weights, values, input_gate,
+                            effective_erase, forget_log_gate, read_indices, read_weights,
+                            output, first, repeated, allocated)
+        if banks and (validate_routes or torch_checks or not state.capacity_is_proven):
+            _run_precheck(layer, shape, dense=False, unique=validate_routes,
+                          capacity=torch_checks or not state.capacity_is_proven, device=device)
+        if not types or not banks:
+            break
+        code = nat.lib().cowsdm_packed_step_floats(layer, shape, types,
+                                                   nat.stream_handle(device))
+        if code != nat.ELIMIT:
+            nat.check(code, "cowsdm_packed_step_floats")
+            break
+        types = 0   # alignment or a row of several passes: widened first
+    if banks and not types:
         nat.check(nat.lib().cowsdm_packed_step(layer, shape, nat.stream_handle(device)),
                   "cowsdm_packed_step")
-    elif allocated is not None:
+    elif not banks and allocated is not None:
         allocated = state.allocated_rows_tensor()
     if reading_dtype != output.dtype:
         output = output.to(reading_dtype)
@@ -1393,21 +1426,35 @@ def dense_sdm_sparse_step(
     _select_backend(backend, tensor=memory, writes=write_indices.shape[1],
                     reads=read_indices.shape[1])
     reading_dtype = values.dtype
-    write_weights, values, input_gate, effective_erase, forget_log_gate, read_weights = (
-        _widen(t) for t in (write_weights, values, input_gate, effective_erase,
-                            forget_log_gate, read_weights))
-    _check_float_tensors((memory, write_weights, values, input_gate, effective_erase,
-                          forget_log_gate, read_weights))
-    index_code = _index_code(write_indices, read_indices)
-    output = torch.empty_like(values)
-    layer = _step_layer(None, memory, write_indices, write_weights, values, input_gate,
-                        effective_erase, forget_log_gate, read_indices, read_weights, output,
-                        None, None, None)
-    shape = _shape(banks, slots, width, write_indices.shape[1], read_indices.shape[1], 1,
-                   index_code)
-    if banks and validate_routes:
-        _run_precheck(layer, shape, dense=True, unique=True, capacity=False, device=device)
-    if banks:
+    writes, reads = write_indices.shape[1], read_indices.shape[1]
+    floats = (write_weights, values, input_gate, effective_erase, forget_log_gate, read_weights)
+    # 16-bit weights, values and gates: as in packed_sdm_cow_step
+    types = _narrow_types(floats, writes=writes, reads=reads, width=width, banks=0)
+    _check_float_tensors((memory,))
+    index_code = None
+    while True:
+        if not types:
+            floats = tuple(_widen(t) for t in floats)
+            _check_float_tensors(floats)
+        write_weights, values, input_gate, effective_erase, forget_log_gate, read_weights = floats
+        if index_code is None:
+            index_code = _index_code(write_indices, read_indices)
+        output = torch.empty_like(values)
+        layer = _step_layer(None, memory, write_indices, write_weights, values, input_gate,
+                            effective_erase, forget_log_gate, read_indices, read_weights,
+                            output, None, None, None)
+        shape = _shape(banks, slots, width, writes, reads, 1, index_code)
+        if banks and validate_routes:
+            _run_precheck(layer, shape, dense=True, unique=True, capacity=False, device=device)
+        if not types or not banks:
+            break
+        code = nat.lib().cowsdm_dense_step_floats(layer, shape, types,
+                                                  nat.stream_handle(device))
+        if code != nat.ELIMIT:
+            nat.check(code, "cowsdm_dense_step_floats")
+            break
+        types = 0
+    if banks and not types:
         nat.check(nat.lib().cowsdm_dense_step(layer, shape, nat.stream_handle(device)),
                   "cowsdm_dense_step")
     return output if reading_dtype == output.dtype else output.to(reading_dtype)

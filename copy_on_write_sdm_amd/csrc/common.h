@@ -95,6 +95,8 @@ struct StepParams {
   int32_t reads;
   int32_t templates;
   int32_t blocks_per_layer;
+  int32_t float_types;           // COWSDM_FLOAT_* of the inputs, two bits at 2k for input k of
+                                 // trace_stride's order (one-step launches of the small kernel)
 };
 
 // ------------------------------------------------------------ wave helpers
@@ -188,6 +190,27 @@ __device__ __forceinline__ void store_row(float* p, const float (&x)[VEC]) {
   } else {
     *p = x[0];
   }
+}
+
+// A float input's element i as loaded, for widen_float (type: COWSDM_FLOAT_*).
+__device__ __forceinline__ uint32_t load_float_bits(const void* base, int64_t i, int type) {
+  return type == COWSDM_FLOAT32 ? static_cast<const uint32_t*>(base)[i]
+                                : static_cast<const uint16_t*>(base)[i];
+}
+
+// Its value in float32, exact.
+__device__ __forceinline__ float widen_float(uint32_t bits, int type) {
+  if (type == COWSDM_FLOAT32) return __uint_as_float(bits);
+  if (type == COWSDM_BFLOAT16) return __uint_as_float(bits << 16);
+  return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(bits)));
+}
+
+// x in 16 bits, rounded to nearest even (NaN stays NaN).
+__device__ __forceinline__ uint16_t narrow_float(float x, int type) {
+  if (type != COWSDM_BFLOAT16) return __builtin_bit_cast(uint16_t, static_cast<_Float16>(x));
+  const uint32_t bits = __float_as_uint(x);
+  if (x != x) return 0x7fc0u;
+  return static_cast<uint16_t>((bits + 0x7fffu + ((bits >> 16) & 1u)) >> 16);
 }
 
 __device__ __forceinline__ uint64_t atomic_load_u64(const int64_t* p) {

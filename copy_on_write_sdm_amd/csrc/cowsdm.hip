@@ -860,7 +860,8 @@ int persistent_vec(int vec, const cowsdm_layer_t* layers, const cowsdm_shape_t* 
 
 int32_t run_step(const cowsdm_layer_t* layers, int32_t nlayers,
                  const cowsdm_shape_t* shape, bool dense, hipStream_t stream,
-                 const cowsdm_trace_t* trace = nullptr, int32_t steps = 1) {
+                 const cowsdm_trace_t* trace = nullptr, int32_t steps = 1,
+                 int32_t float_types = 0) {
   if (int32_t e = check_shape(shape)) return e;
   if (!layers || nlayers <= 0) return fail(COWSDM_EARG, "no layers given");
   for (int32_t i = 0; i < nlayers; ++i) {
@@ -871,6 +872,19 @@ int32_t run_step(const cowsdm_layer_t* layers, int32_t nlayers,
     return fail(COWSDM_EARG, "templates must be positive");
   }
   int vec = row_vec(layers, nlayers, shape, dense, trace);
+  if (float_types) {
+    // 16-bit floats are widened by the small one-step kernel only
+    for (int k : {1, 2, 3, 4, 5, 7}) {
+      if (((float_types >> (2 * k)) & 3) > COWSDM_BFLOAT16) {
+        return fail(COWSDM_EARG, "step: unknown float type");
+      }
+    }
+    if (shape->writes > 4 || shape->reads > 16 || shape->width > kWave * vec ||
+        (!dense && shape->banks > 256)) {
+      return fail(COWSDM_ELIMIT, "16-bit floats: steps need W <= 4, R <= 16, one row pass "
+                                 "(D <= %d here) and packed at most 256 banks", kWave * vec);
+    }
+  }
   if (!dense) {
     // paged slot maps run the small one-step kernel only
     for (int32_t i = 0; i < nlayers; ++i) {
@@ -943,6 +957,7 @@ int32_t run_step(const cowsdm_layer_t* layers, int32_t nlayers,
   P.plan_steps = planned ? trace->scan_steps : 0;
   P.report = persistent ? trace->report : nullptr;
   P.count_table = 0;
+  P.float_types = float_types;
   P.steps = steps;
   for (int k = 0; k < 9; ++k) P.trace_stride[k] = trace ? trace->stride_bytes[k] : 0;
   P.banks = static_cast<int32_t>(shape->banks);
@@ -1402,6 +1417,16 @@ int64_t cowsdm_workspace_bytes(int64_t entries, int64_t capacity_rows) {
 int32_t cowsdm_packed_step(const cowsdm_layer_t* layer, const cowsdm_shape_t* shape,
                            void* stream) {
   return run_step(layer, 1, shape, false, as_stream(stream));
+}
+
+int32_t cowsdm_packed_step_floats(const cowsdm_layer_t* layer, const cowsdm_shape_t* shape,
+                                  int32_t float_types, void* stream) {
+  return run_step(layer, 1, shape, false, as_stream(stream), nullptr, 1, float_types);
+}
+
+int32_t cowsdm_dense_step_floats(const cowsdm_layer_t* layer, const cowsdm_shape_t* shape,
+                                 int32_t float_types, void* stream) {
+  return run_step(layer, 1, shape, true, as_stream(stream), nullptr, 1, float_types);
 }
 
 int32_t cowsdm_packed_step_layers(const cowsdm_layer_t* layers, int32_t nlayers,

@@ -444,7 +444,12 @@ __device__ __forceinline__ void store_paged(const cowsdm_layer_t& L, int64_t ban
 // routes are invalid (index outside [0, N), map entry outside the slab)
 // keeps its writes and returns a zero reading.  Both set the sticky error
 // word.
-template <typename IDX, int VEC, bool DENSE>
+//
+// NARROW: weights, values and gates may be 16-bit floats (P.float_types); they
+// are widened here, after all of them are on their way, and the reading is
+// narrowed to the values' type.  Widening them first took a launch for each:
+// 64 us per call of a bfloat16 model's one-layer step (96 banks), 24 so.
+template <typename IDX, int VEC, bool DENSE, bool NARROW>
 __global__ __launch_bounds__(kStepThreads) void sdm_step_small_kernel(StepParams P) {
   const int layer_id = blockIdx.x / P.blocks_per_layer;
   const int bank = __builtin_amdgcn_readfirstlane(
@@ -458,14 +463,17 @@ __global__ __launch_bounds__(kStepThreads) void sdm_step_small_kernel(StepParams
     return static_cast<const char*>(base) + trace_s * P.trace_stride[k];
   };
   const void* const write_indices = step_ptr(L.write_indices, 0);
-  const float* const write_weights = reinterpret_cast<const float*>(step_ptr(L.write_weights, 1));
-  const float* const step_values = reinterpret_cast<const float*>(step_ptr(L.step_values, 2));
-  const float* const input_gate = reinterpret_cast<const float*>(step_ptr(L.input_gate, 3));
-  const float* const erase_gate = reinterpret_cast<const float*>(step_ptr(L.erase_gate, 4));
-  const float* const forget_gate = reinterpret_cast<const float*>(step_ptr(L.forget_log_gate, 5));
+  const void* const write_weights = step_ptr(L.write_weights, 1);
+  const void* const step_values = step_ptr(L.step_values, 2);
+  const void* const input_gate = step_ptr(L.input_gate, 3);
+  const void* const erase_gate = step_ptr(L.erase_gate, 4);
+  const void* const forget_gate = step_ptr(L.forget_log_gate, 5);
   const void* const read_indices = step_ptr(L.read_indices, 6);
-  const float* const read_weights = reinterpret_cast<const float*>(step_ptr(L.read_weights, 7));
-  float* const output = const_cast<float*>(reinterpret_cast<const float*>(step_ptr(L.output, 8)));
+  const void* const read_weights = step_ptr(L.read_weights, 7);
+  void* const output = const_cast<char*>(step_ptr(L.output, 8));
+  auto float_type = [&](int k) __attribute__((always_inline)) {
+    return NARROW ? (P.float_types >> (2 * k)) & 3 : COWSDM_FLOAT32;
+  };
 
   const int N = P.slots;
   const int D = P.width;
@@ -480,13 +488,14 @@ __global__ __launch_bounds__(kStepThreads) void sdm_step_small_kernel(StepParams
   const int r_of_lane = lane - kSmallReadLane;
   const bool is_r = r_of_lane >= 0 && r_of_lane < R;
   int slot = 0;
-  float weight = 0.0f;
+  uint32_t weight_bits = 0;
   int werr = 0;   // this lane's errors on the write side (skip the bank)
   int rerr = 0;   // ... on the read side (zero reading)
   if (is_w || is_r) {
     const int64_t x = is_w ? load_index<IDX>(write_indices, b * W + lane)
                            : load_index<IDX>(read_indices, b * R + r_of_lane);
-    weight = is_w ? write_weights[b * W + lane] : read_weights[b * R + r_of_lane];
+    weight_bits = is_w ? load_float_bits(write_weights, b * W + lane, float_type(1))
+                       : load_float_bits(read_weights, b * R + r_of_lane, float_type(7));
     if (x < 0 || x >= N) {
       if (is_w) werr |= COWSDM_ERR_WRITE_INDEX;
       else rerr |= COWSDM_ERR_READ_INDEX;
@@ -494,15 +503,29 @@ __global__ __launch_bounds__(kStepThreads) void sdm_step_small_kernel(StepParams
       slot = static_cast<int>(x);
     }
   }
-  const float forget = forget_gate[b];
-  const float in_gate = input_gate[b];
-  const float er_gate = erase_gate[b];
+  const uint32_t forget_bits = load_float_bits(forget_gate, b, float_type(5));
+  const uint32_t in_gate_bits = load_float_bits(input_gate, b, float_type(3));
+  const uint32_t er_gate_bits = load_float_bits(erase_gate, b, float_type(4));
   float vin[VEC];
+  uint32_t vin_bits[VEC];
 #pragma unroll
-  for (int v = 0; v < VEC; ++v) vin[v] = 0.0f;
+  for (int v = 0; v < VEC; ++v) {
+    vin[v] = 0.0f;
+    vin_bits[v] = 0;
+  }
   const int col = lane * VEC;
   const bool col_ok = col < D;
-  if (col_ok) load_row<VEC>(step_values + b * D + col, vin);
+  const bool wide_values = float_type(2) == COWSDM_FLOAT32;
+  if (col_ok) {
+    if (wide_values) {
+      load_row<VEC>(static_cast<const float*>(step_values) + b * D + col, vin);
+    } else {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        vin_bits[v] = load_float_bits(step_values, b * D + col + v, float_type(2));
+      }
+    }
+  }
 
   int64_t tmpl = 0;
   int64_t old_free = 0;
@@ -519,6 +542,14 @@ __global__ __launch_bounds__(kStepThreads) void sdm_step_small_kernel(StepParams
       report_refusal(P, layer_id, bank, lane, trace_s, old_free);
       return;
     }
+  }
+  const float weight = widen_float(weight_bits, is_w ? float_type(1) : float_type(7));
+  const float forget = widen_float(forget_bits, float_type(5));
+  const float in_gate = widen_float(in_gate_bits, float_type(3));
+  const float er_gate = widen_float(er_gate_bits, float_type(4));
+  if (!wide_values) {
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) vin[v] = widen_float(vin_bits[v], float_type(2));
   }
   const int64_t C = pr.capacity;
 
@@ -694,7 +725,16 @@ __global__ __launch_bounds__(kStepThreads) void sdm_step_small_kernel(StepParams
 
   // ---- stores: the reading, the updated rows (a first touch at its popped
   // row), then (packed) the map entries once the launch's tables are built
-  if (col_ok) store_row<VEC>(output + b * D + col, acc);
+  if (col_ok) {
+    if (wide_values) {
+      store_row<VEC>(static_cast<float*>(output) + b * D + col, acc);
+    } else {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        static_cast<uint16_t*>(output)[b * D + col + v] = narrow_float(acc[v], float_type(2));
+      }
+    }
+  }
   const bool commit = wok && fits;
   if (DENSE ? wok : commit) {
 #pragma unroll
@@ -1164,8 +1204,9 @@ void launch_step(const StepParams& P, int blocks, hipStream_t stream) {
 
 template <typename IDX, int VEC, bool DENSE>
 void launch_small(const StepParams& P, int blocks, hipStream_t stream) {
-  hipLaunchKernelGGL((sdm_step_small_kernel<IDX, VEC, DENSE>), dim3(blocks),
-                     dim3(kStepThreads), 0, stream, P);
+  auto* const kernel = P.float_types ? &sdm_step_small_kernel<IDX, VEC, DENSE, true>
+                                     : &sdm_step_small_kernel<IDX, VEC, DENSE, false>;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kStepThreads), 0, stream, P);
 }
 
 template <typename IDX, int MAXW, bool DENSE>

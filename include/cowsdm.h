@@ -285,6 +285,26 @@ int64_t cowsdm_workspace_bytes(int64_t entries, int64_t capacity_rows);
 int32_t cowsdm_packed_step(const cowsdm_layer_t* layer,
                            const cowsdm_shape_t* shape, void* stream);
 
+/* cowsdm_packed_step and cowsdm_dense_step with weights, values and gates in
+ * 16-bit floats, as a half-precision model hands them over (both reference
+ * backends widen them to float32: the kernels on load, allocator.py:74-229,
+ * the torch path with .float(), 1490-1498).  float_types holds a
+ * COWSDM_FLOAT32 / COWSDM_FLOAT16 / COWSDM_BFLOAT16 code, two bits each, at
+ * bit 2k of: write_weights k = 1, step_values 2, input_gate 3, erase_gate 4,
+ * forget_log_gate 5, read_weights 7 (0: all float32).  The reading is written
+ * in step_values' type, rounded to nearest even.  COWSDM_ELIMIT, with nothing
+ * launched, beyond W <= 4, R <= 16, a row one wave covers (D <= 256) and, for
+ * packed state, 256 banks. */
+#define COWSDM_FLOAT32 0
+#define COWSDM_FLOAT16 1
+#define COWSDM_BFLOAT16 2
+int32_t cowsdm_packed_step_floats(const cowsdm_layer_t* layer,
+                                  const cowsdm_shape_t* shape, int32_t float_types,
+                                  void* stream);
+int32_t cowsdm_dense_step_floats(const cowsdm_layer_t* layer,
+                                 const cowsdm_shape_t* shape, int32_t float_types,
+                                 void* stream);
+
 /* The same step for `nlayers` independent layers in one launch (all layers
  * share one shape).  No counterpart in the reference: a batched form of
  * cowsdm_packed_step for callers that already hold every layer's routes. */
