@@ -10,6 +10,503 @@
 //   memory[n]  += write_routes[b, t, n] * delta
 //   readings[b, t] = sum_n read_routes[b, t, n] * memory[n]
 //
+// The route vectors come from product keys: a few of their N entries are not
+// zero.  Producer waves compact every vector to its nonzero entries while the
+// tokens before it run, and the recurrence then touches only those rows, as
+// in route_recurrence.hip (the table of 32 columns in LDS, 8 lanes to a
+// column, the same pipeline).  A vector with more than 8 nonzero write or 32
+// nonzero read routes makes its token a dense one: every row, lane g of a
+// column the rows g, g + 8, ....  A token's arithmetic depends on its own
+// vectors only, so later tokens never change earlier results.  (A zero route
+// times a non-finite row, or a zero route times a non-finite delta, is NaN in
+// the dense sums: every lane starts its sums from 0 * the rows it loaded or
+// wrote, and a delta that is not finite takes every row of its column.)
+//
+// A dense token costs 5.7 us here (N = 256) and 0.8 us with the memory in
+// registers, so a sequence whose first token is dense is left to a kernel
+// that holds it so (below): both are launched, and each takes its sequences.
+// The first token alone decides, which keeps a prefix's results its own.
+//
+// Per-token memories (the backward's input) are 4 N D bytes a token, written
+// by four waves of their own from LDS, 16 bytes a lane and a table row's 32
+// columns (128 bytes) together, between two barriers of the token; the
+// compute waves load the next token's rows and sum the reading meanwhile.
+// (From the compute waves, each storing its 8 columns, 64 batch rows of 64
+// tokens took 210 us against 114: half-written 64-byte requests.)
+//
+// Measured at T = 128, N = 256, D = 128, 4 writes, 16 reads, before (every
+// row of every token in registers) and after, time of the call: with the
+// per-token memories B = 16 275 -> 98 us (269 MB: 2.7 TB/s; what bounds it is
+// the token's two barriers, 0.6 us a token, the bytes alone are 40 us), B = 64
+// and T = 64 338 -> 114 us (537 MB, 4.7 TB/s: the bytes); without them 101 ->
+// 35 us (the token's serial chain and the host's part of the call).  The
+// second launch, where it has nothing to do, costs 3-5 us, 20 at B = 64, N =
+// 1024, D = 256.
+
+#include <type_traits>
+
+#include "lds_recurrence.h"
+
+namespace cowsdm_impl {
+
+constexpr int kDrWrites = kRrGroups;         // nonzero write routes of a sparse token
+constexpr int kDrReads = 4 * kRrGroups;      // nonzero read routes
+constexpr int kDrStoreThreads = 4 * kWave;   // waves that write the per-token memories
+constexpr int kDrProducers = 8 * kWave;      // threads that compact the tokens
+constexpr int kDrThreads = kRrWaves * kWave + kDrProducers;
+constexpr int kDrShift = 4, kDrChunk = 1 << kDrShift;   // tokens staged at a time
+constexpr int kDrCopy = 8;                   // rows of a memory such a thread has in flight
+constexpr int kDrSegments = kRrMaxSlots / kWave;
+constexpr int kCus = 256;
+
+struct RecParams {
+  int64_t batch, time;
+  int slots, width;
+  int blocks;            // column blocks per batch row
+  bool all_dense;        // every sequence is taken as one of dense tokens
+  const float* m0;       // [B, N, D]
+  const float* wr;       // [B, T, N]
+  const float* values;   // [B, T, D]
+  const float* ig;       // [B, T]
+  const float* eg;       // [B, T]
+  const float* flg;      // [B, T]
+  const float* rr;       // [B, T, N]
+  float* readings;       // [B, T, D]
+  float* states;         // [B, T, N, D] or null
+  float* final_memory;   // [B, N, D] or null
+};
+
+// Whether a sequence is one of sparse tokens, by its first token's vectors
+// (the same in every wave that asks).
+__device__ __forceinline__ bool sparse_sequence(const float* w, const float* r, int N) {
+  const int lane = static_cast<int>(threadIdx.x) % kWave;
+  int writes = 0, reads = 0;
+#pragma unroll 4
+  for (int n = lane; n < ((N + kWave - 1) & -kWave); n += kWave) {
+    const int at = n < N ? n : 0;
+    const float x = w[at], y = r[at];
+    writes += __popcll(__ballot(n < N && x != 0.0f));
+    reads += __popcll(__ballot(n < N && y != 0.0f));
+  }
+  return writes <= kDrWrites && reads <= kDrReads;
+}
+
+// A barrier of the workgroup that orders LDS only: global loads and stores
+// stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// V: floats per access to the memories, 4 when D % 4 == 0 and they are
+// 16-byte aligned.  SEG: 64-slot segments of a route vector, at most.
+template <int V, int SEG, bool STATES>
+__global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void recurrence_kernel(RecParams P) {
+  using Rec = RrRecord<1, 4>;
+  using Vec = typename std::conditional<V == 4, float4, float>::type;
+  extern __shared__ char lds[];
+  const int64_t local = blockIdx.x / kXcds;
+  const int64_t b = blockIdx.x % kXcds + kXcds * (local / P.blocks);
+  if (b >= P.batch) return;   // the whole workgroup
+  const int block = static_cast<int>(local % P.blocks);
+  const int nw = (static_cast<int>(blockDim.x) - kDrProducers -
+                  (STATES ? kDrStoreThreads : 0)) / kWave;   // compute waves
+  const int cols = nw * kRrCols;
+  const int N = P.slots, D = P.width, CH = kDrChunk;
+  const int64_t T = P.time;
+  // the whole workgroup again: every wave counts the same vectors
+  if (T > 0 && !sparse_sequence(P.wr + b * T * N, P.rr + b * T * N, N)) return;
+  const int tid = static_cast<int>(threadIdx.x);
+  const int lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int table_bytes = (N + 1) * kRrRowBytes;   // a wave's table, row N unused by routes
+  char* const stage = lds + nw * table_bytes;
+  float* const poison = reinterpret_cast<float*>(stage + 2 * (CH + kRrPad) * Rec::kBytes);
+  const int d0 = block * cols;
+
+  // the workgroup's columns of a [N, D] memory: V floats a thread
+  const int per_row = cols / V;
+  auto table_at = [&](int n, int c) __attribute__((always_inline)) {
+    return reinterpret_cast<Vec*>(lds + (c / kRrCols) * table_bytes + n * kRrRowBytes +
+                                  (c % kRrCols) * 4);
+  };
+  // 0 or NaN per column: whether the initial memory holds a non-finite value
+  if (tid < cols) poison[tid] = 0.0f;
+  __syncthreads();
+  {
+    const float* const m0 = P.m0 + b * N * static_cast<int64_t>(D);
+    const int at_once = static_cast<int>(blockDim.x) / per_row;
+    const int tn = tid / per_row, tc = (tid - tn * per_row) * V;
+    for (int n0 = tn; n0 < N + 1; n0 += kRrRowsAhead * at_once) {
+      Vec v[kRrRowsAhead] = {};
+#pragma unroll
+      for (int q = 0; q < kRrRowsAhead; ++q) {
+        const int n = n0 + q * at_once;
+        if (tn < at_once && d0 + tc < D && n < N) {
+          v[q] = *reinterpret_cast<const Vec*>(m0 + static_cast<int64_t>(n) * D + d0 + tc);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < kRrRowsAhead; ++q) {
+        const int n = n0 + q * at_once;
+        if (tn < at_once && n < N + 1) *table_at(n, tc) = v[q];
+        const float* const e = reinterpret_cast<const float*>(&v[q]);
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+          if (!(e[k] * 0.0f == 0.0f)) poison[tc + k] = __builtin_nanf("");
+        }
+      }
+    }
+  }
+
+  const int64_t chunks = (T + CH - 1) >> kDrShift;
+  const int col = lane / kRrGroups, g = lane % kRrGroups;
+  if (wave >= nw && wave < nw + kDrProducers / kWave) {
+    // ---- producers: wave pw takes the tokens pw, pw + 8, ..., kAhead of them
+    // loaded before they are needed.  A token is compacted in parts, one
+    // beside each of eight tokens, so that none is long beside a token.
+    const int pw = wave - nw;
+    constexpr int kEach = kDrProducers / kWave, kParts = 8;
+    constexpr int kAhead = SEG <= 4 ? 2 : 1;   // divides the tokens of a wave in a chunk
+    float w[kAhead][SEG], r[kAhead][SEG];
+    float value[kAhead] = {}, gate[kAhead] = {}, erase[kAhead] = {}, forget[kAhead] = {};
+    auto load = [&](int i, int64_t t) __attribute__((always_inline)) {
+      if (t >= T) return;
+      const float* const wt = P.wr + (b * T + t) * N;
+      const float* const rt = P.rr + (b * T + t) * N;
+#pragma unroll
+      for (int q = 0; q < SEG; ++q) {
+        const int n = q * kWave + lane;
+        w[i][q] = n < N ? wt[n] : 0.0f;
+        r[i][q] = n < N ? rt[n] : 0.0f;
+      }
+      const int64_t at = b * T + t;
+      value[i] = lane < cols && d0 + lane < D ? P.values[at * D + d0 + lane] : 0.0f;
+      gate[i] = P.ig[at];
+      erase[i] = P.eg[at];
+      forget[i] = P.flg[at];
+    };
+    const uint64_t below = (uint64_t{1} << lane) - 1;
+    char* rec = nullptr;
+    int writes = 0, reads = 0;
+    auto blank = [&]() __attribute__((always_inline)) {   // row N with weight 0 changes nothing
+      if (lane < kDrWrites + kDrReads) {
+        *reinterpret_cast<uint2*>(rec + 8 * lane) =
+            make_uint2(static_cast<uint32_t>(N) * kRrRowBytes, 0u);
+      }
+    };
+    auto compact = [&](float x, int n, int offset, int most, int& count)
+        __attribute__((always_inline)) {
+      const uint64_t some = __ballot(x != 0.0f);
+      const int at = count + __popcll(some & below);
+      if (x != 0.0f && at < most) {
+        *reinterpret_cast<uint2*>(rec + offset + 8 * at) =
+            make_uint2(static_cast<uint32_t>(n) * kRrRowBytes, __float_as_uint(x));
+      }
+      count += __popcll(some);
+    };
+    // part p of token t in slot i: its entries, in order of their rows, over
+    // blank ones; then its gates and value, and the loads of token t + 8 kAhead
+    auto produce = [&](int i, int p, int64_t t) __attribute__((always_inline)) {
+      if (p == 0) {
+        rec = stage + (((t >> kDrShift) & 1) * (CH + kRrPad) + (t & (CH - 1))) * Rec::kBytes;
+        blank();
+        writes = reads = 0;
+      }
+      const bool in = t < T;
+      if (in) {
+#pragma unroll
+        for (int e = p * 2 * SEG / kParts; e < (p + 1) * 2 * SEG / kParts; ++e) {
+          const int q = e / 2;
+          if (e % 2 == 0) {
+            compact(w[i][q], q * kWave + lane, Rec::kWrite, kDrWrites, writes);
+          } else {
+            compact(r[i][q], q * kWave + lane, Rec::kRead, kDrReads, reads);
+          }
+        }
+      }
+      if (p < kParts - 1) return;
+      const float flag = writes > kDrWrites || reads > kDrReads ? 1.0f : 0.0f;
+      if (lane == 0) {
+        *reinterpret_cast<float4*>(rec + Rec::kGates) =
+            in ? make_float4(expf(forget[i]), gate[i], erase[i], flag)
+               : make_float4(1.0f, 0.0f, 0.0f, 0.0f);
+      }
+      if (lane < kRrCols * kRrWaves) {
+        *reinterpret_cast<float*>(rec + Rec::kValue + 4 * lane) = in ? value[i] : 0.0f;
+      }
+      load(i, t + kAhead * kEach);
+    };
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) load(i, pw + i * kEach);
+    for (int q = pw; q < 2 * kRrPad; q += kEach) {   // the records after each stage's chunk
+      rec = stage + ((q / kRrPad) * (CH + kRrPad) + CH + q % kRrPad) * Rec::kBytes;
+      blank();
+      if (lane == 0) {
+        *reinterpret_cast<float4*>(rec + Rec::kGates) = make_float4(1.0f, 0.0f, 0.0f, 0.0f);
+      }
+      if (lane < kRrCols * kRrWaves) *reinterpret_cast<float*>(rec + Rec::kValue + 4 * lane) = 0.0f;
+    }
+    // chunk c of `chunks`, beside chunk c - 1 (whose stage is the other one)
+    auto chunk = [&](int64_t c, bool paced) __attribute__((always_inline)) {
+      for (int j = pw; j < CH; j += kAhead * kEach) {
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+#pragma unroll
+          for (int p = 0; p < kParts; ++p) {
+            if (c < chunks || !paced) produce(i, p, (c << kDrShift) + j + i * kEach);
+            if (paced) {
+              lds_barrier();
+              lds_barrier();
+            }
+          }
+        }
+      }
+    };
+    chunk(0, false);
+    __syncthreads();
+    for (int64_t c = 1; c <= chunks; ++c) {
+      if constexpr (STATES) {
+        chunk(c, true);
+      } else {
+        if (c < chunks) chunk(c, false);
+        __syncthreads();
+      }
+    }
+  } else if (STATES && wave >= nw) {
+    // ---- the per-token memories: the table as it is between a token's barriers
+    const int p = tid - nw * kWave - kDrProducers;
+    const int copiers = kDrStoreThreads / per_row;   // rows at once
+    const int n0 = p / per_row, cc = (p - n0 * per_row) * V;
+    const bool on = n0 < copiers && d0 + cc < D;
+    const int rows = kDrCopy * copiers;
+    typedef float Copy __attribute__((ext_vector_type(V)));
+    float* out = P.states + (b * T * N + n0) * static_cast<int64_t>(D) + d0 + cc;
+    __syncthreads();
+    // (every lane takes part in the barriers, so the loops are the same in all)
+    for (int64_t t = 0; t < chunks << kDrShift; ++t, out += static_cast<int64_t>(N) * D) {
+      lds_barrier();
+      float* to = out;
+      for (int first = 0; first < N; first += rows) {
+        Copy v[kDrCopy];
+#pragma unroll
+        for (int q = 0; q < kDrCopy; ++q) {
+          const int n = first + n0 + q * copiers;
+          v[q] = *reinterpret_cast<const Copy*>(table_at(n < N ? n : N, cc));
+        }
+        if (first + rows >= N) lds_barrier();   // the last rows are in registers
+#pragma unroll
+        for (int q = 0; q < kDrCopy; ++q) {
+          if (on && t < T && first + n0 + q * copiers < N) *reinterpret_cast<Copy*>(to) = v[q];
+          to += static_cast<int64_t>(copiers) * D;
+        }
+      }
+    }
+  } else {
+    // ---- compute waves
+    __syncthreads();
+    char* const mine = lds + wave * table_bytes + col * 4;   // this column's table
+    const int d = d0 + wave * kRrCols + col;
+    float pz = poison[wave * kRrCols + col];   // 0, or NaN once a row was not finite
+    // a token's two barriers: its update is done; its memory has been read out
+    auto updated = [&]() __attribute__((always_inline)) { if (STATES) lds_barrier(); };
+    auto copied = [&]() __attribute__((always_inline)) { if (STATES) lds_barrier(); };
+    auto entry = [&](const char* p) __attribute__((always_inline)) {
+      return *reinterpret_cast<const uint2*>(p);
+    };
+    auto at_row = [&](uint32_t offset) __attribute__((always_inline)) {
+      return reinterpret_cast<float*>(mine + offset);
+    };
+    // a delta that is not finite: zero routes times it are NaN
+    auto spread = [&](float delta) __attribute__((always_inline)) {
+      const bool bad = !(delta * 0.0f == 0.0f);
+      if (__ballot(bad)) {
+        for (int n = g; n < N; n += kRrGroups) {
+          if (bad) *at_row(n * kRrRowBytes) = __builtin_nanf("");
+        }
+      }
+    };
+    for (int64_t c = 0; c < chunks; ++c) {
+      const char* base = stage + (c & 1) * (CH + kRrPad) * Rec::kBytes;
+      const char* pw = base + Rec::kWrite + 8 * g;
+      const char* pr = base + Rec::kRead + 8 * g;
+      const char* pg = base + Rec::kGates;
+      const char* pv = base + Rec::kValue + 4 * (wave * kRrCols + col);
+      // the pipeline: token j's written row, its weight, its decay and its
+      // value before the token; its gates; its read entries; token j - 1's
+      // read weights and rows
+      float* at;
+      float ww, wa, cur, gv;
+      float4 gates;
+      float old_rw[4], old_row[4], old_pz = pz, keep = 0.0f;
+      struct Ahead {
+        uint2 write, read[4];
+        float4 gates;
+        float value;
+      };
+      auto ahead = [&](Ahead& a, int u) __attribute__((always_inline)) {   // iteration u of 8
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a.read[i] = entry(pr + u * Rec::kBytes + 8 * kRrGroups * i);
+        a.write = entry(pw + (u + 1) * Rec::kBytes);
+        a.gates = *reinterpret_cast<const float4*>(pg + (u + 1) * Rec::kBytes);
+        a.value = *reinterpret_cast<const float*>(pv + (u + 1) * Rec::kBytes);
+      };
+      Ahead now_a, next_a;
+      auto begin = [&](int u) __attribute__((always_inline)) {   // token u of the group at p*
+        const uint2 e = entry(pw + u * Rec::kBytes);
+        gates = *reinterpret_cast<const float4*>(pg + u * Rec::kBytes);
+        gv = gates.y * *reinterpret_cast<const float*>(pv + u * Rec::kBytes);
+        at = at_row(e.x);
+        ww = __uint_as_float(e.y);
+        wa = ww != 0.0f ? gates.x : 1.0f;
+        cur = *at;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) old_rw[i] = old_row[i] = 0.0f;
+        ahead(now_a, u);
+      };
+      begin(0);
+      int64_t t = (c << kDrShift) - kRrGroups + g;
+      float* out = P.readings + (b * T + t) * D + d;
+      auto last_reading = [&]() __attribute__((always_inline)) {
+        float sum = old_pz;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum = __builtin_fmaf(old_rw[i], old_row[i], sum);
+        return column_sum8(sum);
+      };
+      for (int j0 = 0; j0 < CH; j0 += kRrGroups) {
+        // lane g: whether token g of these 8 is a dense one
+        const float flag = *reinterpret_cast<const float*>(pg + g * Rec::kBytes + 12);
+        const uint32_t dense = static_cast<uint32_t>(__ballot(flag != 0.0f)) & 0xffu;
+        if (dense == 0) {
+#pragma unroll
+          for (int u = 0; u < kRrGroups; ++u) {
+            ahead(next_a, u + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            cur = cur * wa;
+            const float delta = __builtin_fmaf(-gates.z, column_sum8(__builtin_fmaf(ww, cur, pz)),
+                                               gv);
+            spread(delta);
+            const float now = __builtin_fmaf(ww, delta, cur);
+            *at = now;
+            pz = __builtin_fmaf(now, 0.0f, pz);
+            updated();
+            at = at_row(now_a.write.x);
+            ww = __uint_as_float(now_a.write.y);
+            wa = ww != 0.0f ? now_a.gates.x : 1.0f;
+            cur = *at;
+            float rw[4], row[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              rw[i] = __uint_as_float(now_a.read[i].y);
+              row[i] = *at_row(now_a.read[i].x);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            gates = now_a.gates;
+            gv = now_a.gates.y * now_a.value;
+            now_a = next_a;
+            const float reading = last_reading();
+            keep = g == (u + kRrGroups - 1) % kRrGroups ? reading : keep;
+            if (u == 0 && j0 > 0 && t < T && d < D) *out = keep;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              old_rw[i] = rw[i];
+              old_row[i] = row[i];
+            }
+            old_pz = pz;
+            copied();
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        } else {
+          // one token after the other: the sparse ones in the arithmetic
+          // above, the dense ones over all rows
+          const float before = last_reading();
+          keep = g == kRrGroups - 1 ? before : keep;
+          if (j0 > 0 && t < T && d < D) *out = keep;
+          float reading = 0.0f;
+          for (int u = 0; u < kRrGroups; ++u) {
+            const char* const rec = pw + u * Rec::kBytes;
+            gates = *reinterpret_cast<const float4*>(pg + u * Rec::kBytes);
+            gv = gates.y * *reinterpret_cast<const float*>(pv + u * Rec::kBytes);
+            float sum;
+            if ((dense >> u) & 1u) {
+              const int64_t token = (b * T + (c << kDrShift) + j0 + u) * N;
+              const float* const wt = P.wr + token;
+              const float* const rt = P.rr + token;
+              float part = 0.0f;
+#pragma unroll 8
+              for (int n = g; n < N; n += kRrGroups) {
+                const float w = wt[n];
+                const float m = *at_row(n * kRrRowBytes);
+                part = __builtin_fmaf(w, w != 0.0f ? m * gates.x : m, part);
+              }
+              const float delta = __builtin_fmaf(-gates.z, column_sum8(part), gv);
+              sum = 0.0f;
+#pragma unroll 8
+              for (int n = g; n < N; n += kRrGroups) {
+                const float w = wt[n];
+                float* const p = at_row(n * kRrRowBytes);
+                const float m = *p;
+                const float now = __builtin_fmaf(w, delta, w != 0.0f ? m * gates.x : m);
+                *p = now;
+                pz = __builtin_fmaf(now, 0.0f, pz);
+                sum = __builtin_fmaf(rt[n], now, sum);
+              }
+              updated();
+            } else {
+              const uint2 e = entry(rec);
+              float* const p = at_row(e.x);
+              const float w = __uint_as_float(e.y);
+              const float m = *p * (w != 0.0f ? gates.x : 1.0f);
+              const float delta = __builtin_fmaf(-gates.z,
+                                                 column_sum8(__builtin_fmaf(w, m, pz)), gv);
+              spread(delta);
+              const float now = __builtin_fmaf(w, delta, m);
+              *p = now;
+              pz = __builtin_fmaf(now, 0.0f, pz);
+              updated();
+              sum = pz;
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const uint2 q = entry(pr + u * Rec::kBytes + 8 * kRrGroups * i);
+                sum = __builtin_fmaf(__uint_as_float(q.y), *at_row(q.x), sum);
+              }
+            }
+            reading = column_sum8(sum);
+            keep = g == u ? reading : keep;
+            copied();
+          }
+          // the pipeline again from the next group's first token on; the
+          // last reading is summed once more there, as itself
+          begin(kRrGroups);
+          old_pz = g == 0 ? reading : 0.0f;
+        }
+        pw += kRrGroups * Rec::kBytes;
+        pr += kRrGroups * Rec::kBytes;
+        pg += kRrGroups * Rec::kBytes;
+        pv += kRrGroups * Rec::kBytes;
+        t += kRrGroups;
+        out += kRrGroups * D;
+      }
+      // the chunk's last reading and its last store
+      const float reading = last_reading();
+      keep = g == kRrGroups - 1 ? reading : keep;
+      if (t < T && d < D) *out = keep;
+      if (!STATES) __syncthreads();
+    }
+  }
+  __syncthreads();
+  if (!P.final_memory) return;
+  float* const out = P.final_memory + b * N * static_cast<int64_t>(D);
+  const int at_once = static_cast<int>(blockDim.x) / per_row;
+  const int tn = tid / per_row, tc = (tid - tn * per_row) * V;
+  if (tn >= at_once || d0 + tc >= D) return;
+#pragma unroll 4
+  for (int n = tn; n < N; n += at_once) {
+    *reinterpret_cast<Vec*>(out + static_cast<int64_t>(n) * D + d0 + tc) = *table_at(n, tc);
+  }
+}
+
+// ---- sequences of dense tokens
+//
 // A wave owns 4 columns of one batch row's memory for the whole sequence,
 // in registers: lane = 16 * column + row group, and row group g holds rows
 // g * RPL .. g * RPL + RPL - 1 (RPL rows per lane, N <= 16 * RPL).  A
@@ -23,30 +520,10 @@
 // registers hold; the gates of 64 tokens a lane each, a chunk ahead), and
 // every load is a vector load whose value is first used tokens later.
 
-#include "common.h"
-
-namespace cowsdm_impl {
-
 constexpr int kRecCols = 4;                  // columns per wave
 constexpr int kRecGroups = kWave / kRecCols; // row groups per column: one DPP row
 constexpr int kRecWaves = 4;                 // waves per workgroup
 constexpr int kRecThreads = kRecWaves * kWave;
-constexpr int kRecMaxSlots = 1024;
-
-struct RecParams {
-  int64_t batch, time;
-  int slots, width, col_blocks;
-  const float* m0;       // [B, N, D]
-  const float* wr;       // [B, T, N]
-  const float* values;   // [B, T, D]
-  const float* ig;       // [B, T]
-  const float* eg;       // [B, T]
-  const float* flg;      // [B, T]
-  const float* rr;       // [B, T, N]
-  float* readings;       // [B, T, D]
-  float* states;         // [B, T, N, D] or null
-  float* final_memory;   // [B, N, D] or null
-};
 
 // Sum of v over the 16 lanes of each DPP row, the same value in every lane
 // of the row: an inclusive DPP prefix within the row (row_shr 1, 2, 4, 8;
@@ -118,14 +595,14 @@ constexpr int rec_ahead() {
 
 // EXACT: N == 16 * RPL, every lane's rows are below N (no masks).
 template <int RPL, bool V4, bool EXACT>
-__global__ __launch_bounds__(kRecThreads) void recurrence_kernel(RecParams P) {
+__global__ __launch_bounds__(kRecThreads) void dense_recurrence_kernel(RecParams P) {
   constexpr int PF = rec_ahead<RPL>();
   const int lane = static_cast<int>(threadIdx.x) % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
   const int64_t item = static_cast<int64_t>(blockIdx.x) * kRecWaves + wave;
-  if (item >= P.batch * P.col_blocks) return;
-  const int64_t b = item / P.col_blocks;
-  const int cb = static_cast<int>(item - b * P.col_blocks);
+  if (item >= P.batch * P.blocks) return;
+  const int64_t b = item / P.blocks;
+  const int cb = static_cast<int>(item - b * P.blocks);
   const int col = lane / kRecGroups;
   const int g = lane % kRecGroups;
   const int N = P.slots, D = P.width;
@@ -133,6 +610,7 @@ __global__ __launch_bounds__(kRecThreads) void recurrence_kernel(RecParams P) {
   const int d = cb * kRecCols + col;
   const bool col_ok = d < D;
   const int n0 = g * RPL;
+  if (!P.all_dense && sparse_sequence(P.wr + b * T * N, P.rr + b * T * N, N)) return;
 
   // the lane's rows in a [N, D] block: offset n0 * D + d, stride D (the
   // host keeps N * D below 2^31)
@@ -258,27 +736,91 @@ __global__ __launch_bounds__(256) void dense_routes_kernel(const float* weights,
 }
 
 template <int RPL>
-void launch_recurrence(const RecParams& P, bool v4, unsigned grid, hipStream_t s) {
+void launch_dense_recurrence(const RecParams& P, bool v4, unsigned grid, hipStream_t s) {
   const bool exact = P.slots == kRecGroups * RPL;
   if constexpr (RPL >= 4) {
     if (v4 && exact) {
-      hipLaunchKernelGGL((recurrence_kernel<RPL, true, true>), dim3(grid), dim3(kRecThreads), 0,
+      hipLaunchKernelGGL((dense_recurrence_kernel<RPL, true, true>), dim3(grid), dim3(kRecThreads), 0,
                          s, P);
       return;
     }
     if (v4) {
-      hipLaunchKernelGGL((recurrence_kernel<RPL, true, false>), dim3(grid), dim3(kRecThreads), 0,
+      hipLaunchKernelGGL((dense_recurrence_kernel<RPL, true, false>), dim3(grid), dim3(kRecThreads), 0,
                          s, P);
       return;
     }
   }
   if (exact) {
-    hipLaunchKernelGGL((recurrence_kernel<RPL, false, true>), dim3(grid), dim3(kRecThreads), 0,
+    hipLaunchKernelGGL((dense_recurrence_kernel<RPL, false, true>), dim3(grid), dim3(kRecThreads), 0,
                        s, P);
   } else {
-    hipLaunchKernelGGL((recurrence_kernel<RPL, false, false>), dim3(grid), dim3(kRecThreads), 0,
+    hipLaunchKernelGGL((dense_recurrence_kernel<RPL, false, false>), dim3(grid), dim3(kRecThreads), 0,
                        s, P);
   }
+}
+
+int32_t launch_dense_sequences(RecParams P, hipStream_t s) {
+  P.blocks = (P.width + kRecCols - 1) / kRecCols;
+  const int64_t waves = P.batch * P.blocks;
+  const int64_t grid = (waves + kRecWaves - 1) / kRecWaves;
+  if (grid > (int64_t{1} << 31) - 1) return fail(COWSDM_ELIMIT, "recurrence: batch too large");
+  const int groups_rows = (P.slots + kRecGroups - 1) / kRecGroups;   // rows per lane needed
+  const uintptr_t align = reinterpret_cast<uintptr_t>(P.wr) | reinterpret_cast<uintptr_t>(P.rr);
+  const bool v4 = P.slots % 4 == 0 && align % 16 == 0;
+  const unsigned g = static_cast<unsigned>(grid);
+  if (groups_rows <= 1) {
+    launch_dense_recurrence<1>(P, v4, g, s);
+  } else if (groups_rows <= 2) {
+    launch_dense_recurrence<2>(P, v4, g, s);
+  } else if (groups_rows <= 4) {
+    launch_dense_recurrence<4>(P, v4, g, s);
+  } else if (groups_rows <= 8) {
+    launch_dense_recurrence<8>(P, v4, g, s);
+  } else if (groups_rows <= 16) {
+    launch_dense_recurrence<16>(P, v4, g, s);
+  } else if (groups_rows <= 32) {
+    launch_dense_recurrence<32>(P, v4, g, s);
+  } else {
+    launch_dense_recurrence<64>(P, v4, g, s);
+  }
+  return launch_status("recurrence");
+}
+
+template <int V, int SEG, bool STATES>
+int32_t launch_recurrence(RecParams& P, hipStream_t s) {
+  auto bytes = [&](int nw) {
+    return nw * (P.slots + 1) * kRrRowBytes + 2 * (kDrChunk + kRrPad) * RrRecord<1, 4>::kBytes +
+           4 * nw * kRrCols;
+  };
+  // the waves that D fills, fewer where the tables and the stage would not
+  // fit in LDS
+  int nw = (P.width + kRrCols - 1) / kRrCols;
+  nw = nw > kRrWaves ? kRrWaves : nw;
+  // with per-token memories two waves where four would leave CUs idle, for a
+  // CU writes 64 bytes a cycle: 98 us against 109 at B = 16, T = 128, N = 256,
+  // D = 128; where four fill the chip their 128-byte rows are the better ones
+  // (265 us against 284 at B = 64, T = 16, N = 1024, D = 256)
+  if (STATES && nw > 2 && P.batch * ((P.width + nw * kRrCols - 1) / (nw * kRrCols)) < kCus) nw = 2;
+  while (nw > 1 && bytes(nw) > kRrLds) --nw;
+  const int lds = bytes(nw);
+  P.blocks = (P.width + nw * kRrCols - 1) / (nw * kRrCols);
+  const int64_t grid = kXcds * ((P.batch + kXcds - 1) / kXcds) * P.blocks;
+  if (grid > (int64_t{1} << 31) - 1) return fail(COWSDM_ELIMIT, "recurrence: batch too large");
+  auto* const kernel = &recurrence_kernel<V, SEG, STATES>;
+  if (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(
+        reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return fail(static_cast<int32_t>(e), "recurrence: %d bytes of LDS", lds);
+  }
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)),
+                     dim3(nw * kWave + kDrProducers + (STATES ? kDrStoreThreads : 0)), lds, s, P);
+  return launch_status("recurrence");
+}
+
+template <int V, bool STATES>
+int32_t launch_recurrence_slots(RecParams& P, hipStream_t s) {
+  if (P.slots <= 4 * kWave) return launch_recurrence<V, 4, STATES>(P, s);
+  return launch_recurrence<V, kDrSegments, STATES>(P, s);
 }
 
 }  // namespace cowsdm_impl
@@ -290,8 +832,8 @@ extern "C" int32_t cowsdm_recurrence_forward(const cowsdm_recurrence_t* r, void*
   if (r->batch < 0 || r->time < 0 || r->slots <= 0 || r->width <= 0) {
     return fail(COWSDM_EARG, "recurrence: invalid sizes");
   }
-  if (r->slots > kRecMaxSlots) {
-    return fail(COWSDM_ELIMIT, "recurrence: at most %d slots", kRecMaxSlots);
+  if (r->slots > kRrMaxSlots) {
+    return fail(COWSDM_ELIMIT, "recurrence: at most %d slots", kRrMaxSlots);
   }
   if (r->width > (int64_t{1} << 24) || r->slots * r->width >= (int64_t{1} << 31)) {
     return fail(COWSDM_ELIMIT, "recurrence: width too large");
@@ -309,7 +851,6 @@ extern "C" int32_t cowsdm_recurrence_forward(const cowsdm_recurrence_t* r, void*
   P.time = r->time;
   P.slots = static_cast<int>(r->slots);
   P.width = static_cast<int>(r->width);
-  P.col_blocks = static_cast<int>((r->width + kRecCols - 1) / kRecCols);
   P.m0 = r->initial_memory;
   P.wr = r->write_routes;
   P.values = r->values;
@@ -320,30 +861,27 @@ extern "C" int32_t cowsdm_recurrence_forward(const cowsdm_recurrence_t* r, void*
   P.readings = r->readings;
   P.states = r->states;
   P.final_memory = r->final_memory;
-  const int64_t waves = P.batch * P.col_blocks;
-  const int64_t grid = (waves + kRecWaves - 1) / kRecWaves;
-  if (grid > (int64_t{1} << 31) - 1) return fail(COWSDM_ELIMIT, "recurrence: batch too large");
-  const int groups_rows = (P.slots + kRecGroups - 1) / kRecGroups;   // rows per lane needed
-  const uintptr_t align = reinterpret_cast<uintptr_t>(P.wr) | reinterpret_cast<uintptr_t>(P.rr);
-  const bool v4 = P.slots % 4 == 0 && align % 16 == 0;
-  const unsigned g = static_cast<unsigned>(grid);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (groups_rows <= 1) {
-    launch_recurrence<1>(P, v4, g, s);
-  } else if (groups_rows <= 2) {
-    launch_recurrence<2>(P, v4, g, s);
-  } else if (groups_rows <= 4) {
-    launch_recurrence<4>(P, v4, g, s);
-  } else if (groups_rows <= 8) {
-    launch_recurrence<8>(P, v4, g, s);
-  } else if (groups_rows <= 16) {
-    launch_recurrence<16>(P, v4, g, s);
-  } else if (groups_rows <= 32) {
-    launch_recurrence<32>(P, v4, g, s);
-  } else {
-    launch_recurrence<64>(P, v4, g, s);
+  const uintptr_t align = reinterpret_cast<uintptr_t>(P.m0) |
+                          reinterpret_cast<uintptr_t>(P.states) |
+                          reinterpret_cast<uintptr_t>(P.final_memory);
+  const bool v4 = P.width % 4 == 0 && align % 16 == 0;
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  // up to 64 slots and few columns the memory in registers is the faster one
+  // with per-token memories (59 us against 82 at B = 1, T = 128, N = 32, 70
+  // against 82 at N = 64; 134 against 84 at N = 128, 104 against 89 at N = 32
+  // with B = 64, D = 128); without them it is not (52 us against 30), but both
+  // calls have to give the same readings.  And the sparse sequences' launch, at
+  // most 16 waves to 16 columns, has to stay below 2^32 threads.
+  P.all_dense = (P.slots <= kWave && P.batch * P.width < 4096) ||
+                (P.batch + kXcds - 1) * ((P.width + 15) / 16) >= (int64_t{1} << 22);
+  if (P.time > 0 || P.all_dense) {
+    const int32_t rc = launch_dense_sequences(P, s);
+    if (rc || P.all_dense) return rc;
   }
-  return launch_status("recurrence");
+  if (P.states) {
+    return v4 ? launch_recurrence_slots<4, true>(P, s) : launch_recurrence_slots<1, true>(P, s);
+  }
+  return v4 ? launch_recurrence_slots<4, false>(P, s) : launch_recurrence_slots<1, false>(P, s);
 }
 
 extern "C" int32_t cowsdm_dense_routes(const float* weights, const void* indices,
