@@ -85,7 +85,7 @@ class FaithfulSDMDecodeState:
     # Requests are named by their index in the batch; request r owns bank
     # r * H + h of a layer with H memory heads.  Index lists are handled on
     # the host (one read of the activity mask per call) and sent to the
-    # device once per layer as the bank list its state operation takes.
+    # device as one bank list for the layers of one head count.
 
     def _position_list(self) -> list[int]:
         """Every live request's decode position, on the host."""
@@ -100,9 +100,24 @@ class FaithfulSDMDecodeState:
             raise AssertionError("SDM serving banks do not divide by batch")
         return heads
 
-    def _bank_list(self, requests: list[int], heads: int) -> torch.Tensor:
-        banks = [request * heads + head for request in requests for head in range(heads)]
-        return torch.tensor(banks, device=self.device, dtype=torch.int64)
+    @staticmethod
+    def _packed(states) -> bool:
+        """Whether a lifecycle operation can take all layers at once: plain
+        packed states, each its own (another class keeps its own methods)."""
+
+        return (all(type(state) is PackedSDMCopyOnWriteState for state in states)
+                and len({id(state) for state in states}) == len(states))
+
+    def _bank_lists(self, requests: list[int], batch: int) -> list[torch.Tensor]:
+        """The banks of ``requests`` in every SDM layer, one tensor for the
+        layers of one head count."""
+
+        lists: dict[int, torch.Tensor] = {}
+        for heads in [self._heads(state, batch) for state in self.sdm_states]:
+            if heads not in lists:
+                banks = [request * heads + head for request in requests for head in range(heads)]
+                lists[heads] = torch.tensor(banks, device=self.device, dtype=torch.int64)
+        return [lists[self._heads(state, batch)] for state in self.sdm_states]
 
     def _requests_to_release(self, sequence_indices) -> list[int]:
         """The requests a release names, in the order given, after checking
@@ -132,10 +147,12 @@ class FaithfulSDMDecodeState:
         requests = self._requests_to_release(sequence_indices)
         if not requests:
             return 0
-        freed = 0
-        for state in self.sdm_states:
-            banks = self._bank_list(requests, self._heads(state, self.batch))
-            freed += int(state.release(banks))
+        banks = self._bank_lists(requests, self.batch)
+        if self._packed(self.sdm_states):
+            released = PackedSDMCopyOnWriteState.release_layers(self.sdm_states, banks)
+            freed = int(torch.stack(released).sum()) if released else 0
+        else:
+            freed = sum(int(state.release(b)) for state, b in zip(self.sdm_states, banks))
         mask = torch.ones(self.batch, dtype=torch.bool)
         mask[requests] = False
         self.active_sequences &= mask.to(self.device)
@@ -150,12 +167,15 @@ class FaithfulSDMDecodeState:
 
         live = self.active_sequences.tolist()
         kept = [r for r, on in enumerate(live) if on]
-        for state in self.sdm_states:
-            if not live:
-                if state.banks:
-                    raise AssertionError("empty serving batch retained SDM banks")
-                continue
-            state.retain_banks(self._bank_list(kept, self._heads(state, len(live))))
+        if live:
+            banks = self._bank_lists(kept, len(live))
+            if self._packed(self.sdm_states):
+                PackedSDMCopyOnWriteState.retain_banks_layers(self.sdm_states, banks)
+            else:
+                for state, b in zip(self.sdm_states, banks):
+                    state.retain_banks(b)
+        elif any(state.banks for state in self.sdm_states):
+            raise AssertionError("empty serving batch retained SDM banks")
         index = torch.tensor(kept, device=self.device, dtype=torch.int64)
         self.dense_keys = tuple(t.index_select(0, index).contiguous() for t in self.dense_keys)
         self.dense_values = tuple(t.index_select(0, index).contiguous()
@@ -187,8 +207,11 @@ class FaithfulSDMDecodeState:
                 and len(self.dense_keys) == len(incoming.dense_keys))
         if not same:
             raise ValueError("admitted faithful-SDM state is incompatible")
-        for mine, theirs in zip(self.sdm_states, incoming.sdm_states):
-            mine.append_banks_from(theirs)
+        if self._packed(self.sdm_states) and self._packed(incoming.sdm_states):
+            PackedSDMCopyOnWriteState.append_banks_layers(self.sdm_states, incoming.sdm_states)
+        else:
+            for mine, theirs in zip(self.sdm_states, incoming.sdm_states):
+                mine.append_banks_from(theirs)
         self.dense_keys = tuple(torch.cat((a, b)).contiguous()
                                 for a, b in zip(self.dense_keys, incoming.dense_keys))
         self.dense_values = tuple(torch.cat((a, b)).contiguous()
