@@ -268,11 +268,12 @@ __global__ void grow_free_kernel(const int32_t* old_free_rows,
 
 __global__ void add_counter_kernel(int32_t* counter, int64_t delta,
                                    const int64_t* delta_ptr, int32_t sign,
-                                   int32_t* clear) {
+                                   int32_t* clear, int64_t* moved) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     const int64_t d = delta_ptr ? *delta_ptr : delta;
     *counter = static_cast<int32_t>(*counter + sign * d);
     if (clear) *clear = 0;
+    if (moved) *moved = d;
   }
 }
 
@@ -549,14 +550,6 @@ __global__ void fill_free_tail_kernel(int32_t* free_rows, int64_t capacity,
   }
 }
 
-__global__ void copy_i32_kernel(int32_t* dst, const int32_t* src, int64_t n) {
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-       i < n; i += stride) {
-    dst[i] = src[i];
-  }
-}
-
 __global__ void gather_banks_kernel(const int32_t* map, const int64_t* tmpl,
                                     int64_t banks, int64_t slots, const int64_t* bank_list,
                                     int64_t nsel, int32_t* new_map,
@@ -588,6 +581,14 @@ __global__ void zero_i64_kernel(int64_t* p, int64_t n) {
        i < n; i += stride) {
     p[i] = 0;
   }
+}
+
+// The check of a bank list starts from nothing marked and no fault.
+__global__ void clear_marks_kernel(int32_t* marks, int64_t banks, int64_t* result) {
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  for (int64_t i = t0; i < banks; i += stride) marks[i] = 0;
+  if (t0 == 0) *result = 0;
 }
 
 __global__ void zero_i32_kernel(int32_t* p, int64_t n) {
@@ -1654,7 +1655,7 @@ int32_t cowsdm_grow(const float* old_values, int64_t old_capacity, float* new_va
   if (int32_t e = launch_status("grow free")) return e;
   hipLaunchKernelGGL(add_counter_kernel, dim3(1), dim3(64), 0, s, free_count,
                      new_capacity - old_capacity, static_cast<const int64_t*>(nullptr), 1,
-                     overflow_flag);
+                     overflow_flag, static_cast<int64_t*>(nullptr));
   return launch_status("grow counter");
 }
 
@@ -1756,15 +1757,10 @@ int32_t cowsdm_append_banks(const int32_t* map, const int64_t* tmpl, int64_t ban
   const hipStream_t s = as_stream(stream);
   const int64_t entries = other_banks * slots;
   Workspace ws = carve(workspace, entries, other_capacity_rows);
-  if (banks > 0) {
-    hipLaunchKernelGGL(copy_i32_kernel, dim3(grid_for(banks * slots, 256)), dim3(256), 0, s,
-                       new_map, map, banks * slots);
-    if (int32_t e = launch_status("append copy map")) return e;
-  }
-  hipLaunchKernelGGL(gather_banks_kernel, dim3(grid_for(banks + other_banks, 256)),
-                     dim3(256), 0, s, static_cast<const int32_t*>(nullptr), tmpl, banks, slots,
-                     static_cast<const int64_t*>(nullptr), banks,
-                     static_cast<int32_t*>(nullptr), new_tmpl, other_tmpl, other_banks);
+  const int64_t moved = banks * slots > banks + other_banks ? banks * slots : banks + other_banks;
+  hipLaunchKernelGGL(gather_banks_kernel, dim3(grid_for(moved, 256)), dim3(256), 0, s, map, tmpl,
+                     banks, slots, static_cast<const int64_t*>(nullptr), banks, new_map, new_tmpl,
+                     other_tmpl, other_banks);
   if (int32_t e = launch_status("append templates")) return e;
   if (entries == 0) return 0;
   RankSource src{other_map, nullptr, nullptr, slots, entries, other_banks};
@@ -1786,7 +1782,8 @@ int32_t cowsdm_append_banks(const int32_t* map, const int64_t* tmpl, int64_t ban
                      other_capacity_rows, width);
   if (int32_t e = launch_status("append copy")) return e;
   hipLaunchKernelGGL(add_counter_kernel, dim3(1), dim3(64), 0, s, free_count, int64_t{0},
-                     static_cast<const int64_t*>(ws.total), -1, static_cast<int32_t*>(nullptr));
+                     static_cast<const int64_t*>(ws.total), -1, static_cast<int32_t*>(nullptr),
+                     static_cast<int64_t*>(nullptr));
   return launch_status("append counter");
 }
 
@@ -1799,13 +1796,9 @@ int32_t cowsdm_check_banks(const int32_t* map, int64_t banks, int64_t slots,
   }
   const hipStream_t s = as_stream(stream);
   Workspace ws = carve(workspace, banks * slots, banks);
-  hipLaunchKernelGGL(zero_i64_kernel, dim3(1), dim3(64), 0, s, result, int64_t{1});
-  if (int32_t e = launch_status("check_banks zero")) return e;
-  if (banks > 0) {
-    hipLaunchKernelGGL(zero_i32_kernel, dim3(grid_for(banks, 256)), dim3(256), 0, s,
-                       ws.list_a, banks);
-    if (int32_t e = launch_status("check_banks marks")) return e;
-  }
+  hipLaunchKernelGGL(clear_marks_kernel, dim3(grid_for(banks, 256)), dim3(256), 0, s, ws.list_a,
+                     banks, result);
+  if (int32_t e = launch_status("check_banks marks")) return e;
   if (nsel > 0) {
     hipLaunchKernelGGL(mark_banks_kernel, dim3(grid_for(nsel, 256)), dim3(256), 0, s,
                        bank_list, nsel, banks, ws.list_a, result);
@@ -1840,11 +1833,9 @@ int32_t cowsdm_release(int32_t* map, int64_t banks, int64_t slots, const int64_t
   a.map_clear = map;
   if (int32_t e = rank_apply(src, ws, a, s)) return e;
   hipLaunchKernelGGL(add_counter_kernel, dim3(1), dim3(64), 0, s, free_count, int64_t{0},
-                     static_cast<const int64_t*>(ws.total), 1, static_cast<int32_t*>(nullptr));
-  if (int32_t e = launch_status("release counter")) return e;
-  hipLaunchKernelGGL(copy_i64_kernel, dim3(1), dim3(64), 0, s, released,
-                     static_cast<const int64_t*>(ws.total), int64_t{1});
-  return launch_status("release count");
+                     static_cast<const int64_t*>(ws.total), 1, static_cast<int32_t*>(nullptr),
+                     released);
+  return launch_status("release counter");
 }
 
 int32_t cowsdm_retain_banks(const int32_t* map, const int64_t* tmpl, int64_t banks,
