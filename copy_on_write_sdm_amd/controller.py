@@ -313,34 +313,36 @@ def decode_sdm_layers_controller(controllers: Sequence[SDMController],
     in one launch.  The layers' states are proven or grow (and prove) here,
     with direct maps (``can_decode_layers``).  The buffers between the kernels
     are one allocation of this call, each in two copies that the layers take
-    in turn."""
+    in turn, at the same place for every layer: the launch that finishes layer
+    i and prepares layer i + 1 reads layer i - 1's sum from the copy that it
+    writes layer i + 1's keys, gates and routes to, and its workgroups are not
+    ordered."""
 
     batch = tokens.shape[0]
     for c in controllers:
         _check_tokens(c, tokens)
     device = tokens.device
     lib, stream = nat.lib(), nat.stream_handle(device)
-    layers, size = [], 0
-    for index, c in enumerate(controllers):
+    layers, floats = [], []
+    for c in controllers:
         banks = batch * c.memory_heads
         reads, writes = c.route_counts()
-        floats = (batch * c.width, banks * c.key_width_per_head, banks * c.key_width_per_head,
-                  batch * c.width, banks, banks, banks * reads, 2 * banks * reads,
-                  banks * writes, 2 * banks * writes, batch * c.width, batch * c.width,
-                  batch * c.width)
-        offsets, at = [], 0
-        for n in floats:
-            offsets.append(at)
-            at += -(-n // 4) * 16        # 16-byte aligned
-        size = max(size, at)
-        layers.append((banks, reads, writes, offsets))
+        layers.append((banks, reads, writes))
+        floats.append((batch * c.width, banks * c.key_width_per_head,
+                       banks * c.key_width_per_head, batch * c.width, banks, banks,
+                       banks * reads, 2 * banks * reads, banks * writes, 2 * banks * writes,
+                       batch * c.width, batch * c.width, batch * c.width))
+    offsets, size = [], 0
+    for n in map(max, zip(*floats)):
+        offsets.append(size)
+        size += -(-n // 4) * 16        # 16-byte aligned
     work = torch.empty(2 * size, device=device, dtype=torch.uint8)
     base = work.data_ptr()
     x = tokens.contiguous()
     result = torch.empty(batch, 1, controllers[0].width, device=device)
 
     def buffers(index: int) -> list[int]:
-        return [base + (index % 2) * size + offset for offset in layers[index][3]]
+        return [base + (index % 2) * size + offset for offset in offsets]
 
     def prepare(index: int, b: list[int]) -> tuple:
         return (b[0], b[1], b[2], b[3], b[4], b[5], controllers[index].reads,
@@ -353,7 +355,7 @@ def decode_sdm_layers_controller(controllers: Sequence[SDMController],
         "cowsdm_controller_prepare_routes")
     last = len(layers) - 1
     for index, (c, st) in enumerate(zip(controllers, states)):
-        banks, reads, writes, _ = layers[index]
+        banks, reads, writes = layers[index]
         if st.banks != banks:
             raise ValueError("packed SDM banks do not match batch and memory heads")
         if st.width != c.head_width:
