@@ -28,9 +28,12 @@
 // 207 us, 0.10 us per token of a bank, where the dense route vectors and the
 // dense-route kernel took 445 + 1,858 us; one bank alone takes 193 us.
 //
-// Non-finite values spread as in the dense sums, where a zero route times a
-// non-finite row is NaN: every lane keeps 0 * (each row it loaded or wrote),
-// 0 or NaN, and starts its partial sums from it.
+// Values that are not finite spread as in the dense sums, where a zero route
+// times such a row, or times such a delta, is NaN.  Every lane keeps 0 * (each
+// row it wrote), 0 or NaN, and starts its partial sums from it, which marks
+// the columns that met one; at the end of the sequence a wave takes its marked
+// columns again from the first token on, one token after the other with all
+// rows looked over, until everything in them is NaN (exact_columns).
 
 #include <type_traits>
 
@@ -55,6 +58,91 @@ struct RrParams {
   float* readings;              // [B * T * H, D]
   float* final_memory;          // [B * H, N, D]
 };
+
+// A wave's columns (of `bad`: the same in a column's lanes) of a bank's table
+// and readings in the dense sums' own terms, from the initial memory `m0` on:
+// as the kernel below computes them, but the rows that a sum has no route for,
+// or a zero one, are looked over for values that are not finite.  Tokens are
+// taken until every row of these columns is NaN: what follows is NaN, and
+// marked columns already read so.  `mine`: the column's table.
+template <int WPL, int RPL>
+__device__ __forceinline__ void exact_columns(const RrParams& P, char* mine, int64_t b, int64_t h,
+                                              int d, int g, bool bad) {
+  const int N = P.slots, D = P.width;
+  const bool in = d < D;
+  const float* const m0 = P.m0 + h * N * static_cast<int64_t>(D);
+  auto row = [&](int n) __attribute__((always_inline)) {
+    return reinterpret_cast<float*>(mine + n * kRrRowBytes);
+  };
+  for (int n = g; n <= N; n += kRrGroups) {
+    if (bad) *row(n) = in && n < N ? m0[static_cast<int64_t>(n) * D + d] : 0.0f;
+  }
+  // 0, or NaN if a row of the column is not finite
+  auto look_over = [&]() __attribute__((always_inline)) {
+    float z = 0.0f;
+#pragma unroll 4
+    for (int n = g; n < N; n += kRrGroups) z = __builtin_fmaf(*row(n), 0.0f, z);
+    return z;
+  };
+  for (int64_t t = 0; t < P.time; ++t) {
+    const int64_t at = (b * P.time + t) * P.heads + h;
+    // the lane's routes; none, or one past the table, has weight 0 and row N
+    auto route = [&](const int64_t* idx, const float* w, int k, int i, float& weight)
+        __attribute__((always_inline)) {
+      const int j = g + kRrGroups * i;
+      const int64_t n = j < k ? idx[at * k + j] : -1;
+      const bool on = n >= 0 && n < N;
+      weight = on ? w[at * k + j] : 0.0f;
+      return row(on ? static_cast<int>(n) : N);
+    };
+    const float alpha = expf(P.forget[at]), gate = P.gate[at];
+    const float gv = gate * (in ? P.values[at * D + d] : 0.0f);
+    float* to[WPL];
+    float ww[WPL], cur[WPL];
+#pragma unroll
+    for (int i = 0; i < WPL; ++i) {
+      to[i] = route(P.write_idx, P.write_w, P.writes, i, ww[i]);
+      cur[i] = *to[i] * alpha;
+    }
+#pragma unroll
+    for (int i = 0; i < WPL; ++i) {
+      if (bad && ww[i] != 0.0f) *to[i] = 0.0f;   // out of the others' sight
+    }
+    float part = look_over();
+#pragma unroll
+    for (int i = 0; i < WPL; ++i) {
+      if (ww[i] != 0.0f) part = __builtin_fmaf(ww[i], cur[i], part);
+    }
+    const float delta = __builtin_fmaf(-gate, column_sum8(part), gv);
+    if (bad && !(delta * 0.0f == 0.0f)) {
+      for (int n = g; n < N; n += kRrGroups) *row(n) = __builtin_nanf("");
+    }
+#pragma unroll
+    for (int i = 0; i < WPL; ++i) {
+      if (bad && ww[i] != 0.0f) *to[i] = __builtin_fmaf(ww[i], delta, cur[i]);
+    }
+    float* from[RPL];
+    float rw[RPL], val[RPL];
+#pragma unroll
+    for (int i = 0; i < RPL; ++i) {
+      from[i] = route(P.read_idx, P.read_w, P.reads, i, rw[i]);
+      val[i] = *from[i];
+    }
+#pragma unroll
+    for (int i = 0; i < RPL; ++i) {
+      if (bad && rw[i] != 0.0f) *from[i] = 0.0f;
+    }
+    float sum = look_over();
+#pragma unroll
+    for (int i = 0; i < RPL; ++i) {
+      if (rw[i] != 0.0f) sum = __builtin_fmaf(rw[i], val[i], sum);
+      if (bad && rw[i] != 0.0f) *from[i] = val[i];
+    }
+    const float reading = column_sum8(sum);
+    if (bad && g == 0) P.readings[at * D + d] = reading;
+    if (__ballot(bad && delta == delta) == 0) break;
+  }
+}
 
 // WPL, RPL: write and read routes per lane (W <= 8 * WPL, R <= 8 * RPL).
 // V: floats per access to the initial and final memory, 4 when D % 4 == 0 and
@@ -124,7 +212,6 @@ __global__ __launch_bounds__(kRrThreads, 4) void route_recurrence_kernel(RrParam
   // meeting at one barrier before the first and one after every chunk
   const int64_t chunks = (T + CH - 1) >> P.chunk_shift;
   const int col = lane / kRrGroups, g = lane % kRrGroups;
-  float spread = 0.0f;   // compute waves: 0, or NaN once a delta was not finite
   if (wave >= nw) {
     // A producer's share of a chunk on its way from memory to the stage: the
     // loads of a chunk are issued a whole chunk before they are stored.
@@ -299,7 +386,6 @@ __global__ __launch_bounds__(kRrThreads, 4) void route_recurrence_kernel(RrParam
             *reinterpret_cast<float*>(at[i]) = now;
             pz = __builtin_fmaf(now, 0.0f, pz);
           }
-          spread = __builtin_fmaf(delta, 0.0f, spread);
 #pragma unroll
           for (int i = 0; i < WPL; ++i) {
             at[i] = mine + now_a.write[i].x;
@@ -349,23 +435,15 @@ __global__ __launch_bounds__(kRrThreads, 4) void route_recurrence_kernel(RrParam
       if (t < T && d < D) *out = keep;
       __syncthreads();
     }
+    const bool bad = d < D && !(column_sum8(pz) == 0.0f);
+    if (__ballot(bad)) exact_columns<WPL, RPL>(P, mine, b, h, d, g, bad);
   }
-  // a delta that is not finite reaches every row of its column in the dense
-  // update (zero route times delta)
-  if (wave < nw && g == 0) poison[wave * kRrCols + col] = spread;
   __syncthreads();
   float* const out = P.final_memory + bank * N * static_cast<int64_t>(D) + d0 + tc;
   if (!tcol) return;
-  float p0[V];
-#pragma unroll
-  for (int k = 0; k < V; ++k) p0[k] = poison[tc + k];
 #pragma unroll 4
   for (int n = tn; n < N; n += rows_at_once) {
-    Vec v = *table_at(n, tc);
-    float* const e = reinterpret_cast<float*>(&v);
-#pragma unroll
-    for (int k = 0; k < V; ++k) e[k] = p0[k] == 0.0f ? e[k] : p0[k];
-    *reinterpret_cast<Vec*>(out + static_cast<int64_t>(n) * D) = v;
+    *reinterpret_cast<Vec*>(out + static_cast<int64_t>(n) * D) = *table_at(n, tc);
   }
 }
 
