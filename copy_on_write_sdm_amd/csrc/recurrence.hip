@@ -17,10 +17,13 @@
 // column, the same pipeline).  A vector with more than 8 nonzero write or 32
 // nonzero read routes makes its token a dense one: every row, lane g of a
 // column the rows g, g + 8, ....  A token's arithmetic depends on its own
-// vectors only, so later tokens never change earlier results.  (A zero route
-// times a non-finite row, or a zero route times a non-finite delta, is NaN in
-// the dense sums: every lane starts its sums from 0 * the rows it loaded or
-// wrote, and a delta that is not finite takes every row of its column.)
+// vectors only, so later tokens never change earlier results.
+//
+// A zero route times a row, or a delta, that is not finite is NaN in the dense
+// sums.  Every lane starts its sums from 0 * the rows it wrote, so a column
+// that met one reads NaN from that token to the last; at the end its wave
+// takes it again with every token a dense one, and stores what follows the
+// first reading that is not finite.
 //
 // A dense token costs 5.7 us here (N = 256) and 0.8 us with the memory in
 // registers, so a sequence whose first token is dense is left to a kernel
@@ -97,6 +100,69 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// A wave's columns that are `bad` (the same in a column's lanes), from the
+// initial memory on with every token a dense one: the table (`mine`: the
+// column's) is left as the final memory, and readings and per-token memories
+// are stored from the first reading that is not finite.
+template <bool STATES>
+__device__ __forceinline__ void redo_columns(const RecParams& P, char* mine, int64_t b, int d,
+                                             int g, bool bad) {
+  const int N = P.slots, D = P.width;
+  const int64_t T = P.time;
+  float* const readings = P.readings + b * T * D + (bad ? d : 0);
+  auto finite = [](float x) __attribute__((always_inline)) { return x * 0.0f == 0.0f; };
+  auto row = [&](int n) __attribute__((always_inline)) {
+    return reinterpret_cast<float*>(mine + n * kRrRowBytes);
+  };
+  __threadfence();   // the wave's own readings, by other lanes of it
+  int64_t from = T;
+  for (int64_t t = g; bad && t < from; t += kRrGroups) {
+    if (!finite(readings[t * D])) from = t;
+  }
+#pragma unroll
+  for (int o = kRrGroups / 2; o > 0; o >>= 1) {
+    const int64_t other = __shfl_xor(from, o, kWave);
+    from = other < from ? other : from;
+  }
+  for (int n = g; n < N; n += kRrGroups) {
+    if (bad) *row(n) = P.m0[(b * N + n) * static_cast<int64_t>(D) + d];
+  }
+  for (int64_t t = 0; t < T; ++t) {
+    const int64_t bt = b * T + t;
+    const float* const wt = P.wr + bt * N;
+    const float* const rt = P.rr + bt * N;
+    const float alpha = expf(P.flg[bt]);
+    float part = 0.0f;
+#pragma unroll 8
+    for (int n = g; n < N; n += kRrGroups) {
+      const float w = wt[n], m = *row(n);
+      part = __builtin_fmaf(w, w != 0.0f ? m * alpha : m, part);
+    }
+    const float gv = P.ig[bt] * (bad ? P.values[bt * D + d] : 0.0f);
+    const float delta = __builtin_fmaf(-P.eg[bt], column_sum8(part), gv);
+    float sum = 0.0f;
+#pragma unroll 8
+    for (int n = g; n < N; n += kRrGroups) {
+      const float w = wt[n], m = *row(n);
+      const float now = __builtin_fmaf(w, delta, w != 0.0f ? m * alpha : m);
+      if (bad) *row(n) = now;
+      sum = __builtin_fmaf(rt[n], now, sum);
+    }
+    const float reading = column_sum8(sum);
+    if (bad && t >= from) {
+      if (g == 0) readings[t * D] = reading;
+      if (STATES) {
+        for (int n = g; n < N; n += kRrGroups) {
+          P.states[(bt * N + n) * static_cast<int64_t>(D) + d] = *row(n);
+        }
+      }
+    }
+    // every row of these columns is NaN, and so is what follows; their
+    // readings are already
+    if (!STATES && __ballot(bad && delta == delta) == 0) break;
+  }
+}
+
 // V: floats per access to the memories, 4 when D % 4 == 0 and they are
 // 16-byte aligned.  SEG: 64-slot segments of a route vector, at most.
 template <int V, int SEG, bool STATES>
@@ -130,7 +196,9 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
                                   (c % kRrCols) * 4);
   };
   // 0 or NaN per column: whether the initial memory holds a non-finite value
+  int* const redo = reinterpret_cast<int*>(poison + cols);   // set: some columns are taken again
   if (tid < cols) poison[tid] = 0.0f;
+  if (tid == 0) *redo = 0;
   __syncthreads();
   {
     const float* const m0 = P.m0 + b * N * static_cast<int64_t>(D);
@@ -160,6 +228,7 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
 
   const int64_t chunks = (T + CH - 1) >> kDrShift;
   const int col = lane / kRrGroups, g = lane % kRrGroups;
+  float pz = 0.0f;   // compute waves: NaN once a row was not finite
   if (wave >= nw && wave < nw + kDrProducers / kWave) {
     // ---- producers: wave pw takes the tokens pw, pw + 8, ..., kAhead of them
     // loaded before they are needed.  A token is compacted in parts, one
@@ -306,7 +375,7 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
     __syncthreads();
     char* const mine = lds + wave * table_bytes + col * 4;   // this column's table
     const int d = d0 + wave * kRrCols + col;
-    float pz = poison[wave * kRrCols + col];   // 0, or NaN once a row was not finite
+    pz = poison[wave * kRrCols + col];
     // a token's two barriers: its update is done; its memory has been read out
     auto updated = [&]() __attribute__((always_inline)) { if (STATES) lds_barrier(); };
     auto copied = [&]() __attribute__((always_inline)) { if (STATES) lds_barrier(); };
@@ -315,15 +384,6 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
     };
     auto at_row = [&](uint32_t offset) __attribute__((always_inline)) {
       return reinterpret_cast<float*>(mine + offset);
-    };
-    // a delta that is not finite: zero routes times it are NaN
-    auto spread = [&](float delta) __attribute__((always_inline)) {
-      const bool bad = !(delta * 0.0f == 0.0f);
-      if (__ballot(bad)) {
-        for (int n = g; n < N; n += kRrGroups) {
-          if (bad) *at_row(n * kRrRowBytes) = __builtin_nanf("");
-        }
-      }
     };
     for (int64_t c = 0; c < chunks; ++c) {
       const char* base = stage + (c & 1) * (CH + kRrPad) * Rec::kBytes;
@@ -384,7 +444,6 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
             cur = cur * wa;
             const float delta = __builtin_fmaf(-gates.z, column_sum8(__builtin_fmaf(ww, cur, pz)),
                                                gv);
-            spread(delta);
             const float now = __builtin_fmaf(ww, delta, cur);
             *at = now;
             pz = __builtin_fmaf(now, 0.0f, pz);
@@ -458,7 +517,6 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
               const float m = *p * (w != 0.0f ? gates.x : 1.0f);
               const float delta = __builtin_fmaf(-gates.z,
                                                  column_sum8(__builtin_fmaf(w, m, pz)), gv);
-              spread(delta);
               const float now = __builtin_fmaf(w, delta, m);
               *p = now;
               pz = __builtin_fmaf(now, 0.0f, pz);
@@ -493,7 +551,18 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
       if (!STATES) __syncthreads();
     }
   }
-  __syncthreads();
+  // a column that was never other than finite keeps pz 0
+  const bool bad = wave < nw && T > 0 && d0 + wave * kRrCols + col < D &&
+                   !(column_sum8(pz) == 0.0f);
+  if (bad) *redo = 1;
+  __syncthreads();   // what the store waves wrote is out, too
+  if (*redo) {
+    if (__ballot(bad)) {
+      redo_columns<STATES>(P, lds + wave * table_bytes + col * 4, b, d0 + wave * kRrCols + col, g,
+                           bad);
+    }
+    __syncthreads();
+  }
   if (!P.final_memory) return;
   float* const out = P.final_memory + b * N * static_cast<int64_t>(D);
   const int at_once = static_cast<int>(blockDim.x) / per_row;
@@ -790,7 +859,7 @@ template <int V, int SEG, bool STATES>
 int32_t launch_recurrence(RecParams& P, hipStream_t s) {
   auto bytes = [&](int nw) {
     return nw * (P.slots + 1) * kRrRowBytes + 2 * (kDrChunk + kRrPad) * RrRecord<1, 4>::kBytes +
-           4 * nw * kRrCols;
+           4 * nw * kRrCols + 4;
   };
   // the waves that D fills, fewer where the tables and the stage would not
   // fit in LDS

@@ -15,6 +15,7 @@ import numpy as np
 import pytest
 import torch
 
+import copy_on_write_sdm_amd as cow
 from copy_on_write_sdm_amd.recurrence import route_recurrence
 from oracle import serial
 
@@ -124,3 +125,58 @@ def test_route_recurrence(device, time, slots, width, writes, reads, planted):
         others = [c for c in range(width) if c != COLUMN]
         assert torch.equal(readings[:, others], before[0][:, others])
         assert torch.equal(final[:, :, others], before[1][:, :, others])
+
+
+@pytest.mark.parametrize("planted", PLANTED)
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("time,slots,width,writes,reads", [
+    (1, 70, 40, 4, 8), (20, 70, 33, 4, 16), (48, 100, 130, 8, 24), (17, 300, 12, 4, 32),
+    (20, 32, 16, 4, 8)])
+def test_dense_route_recurrence(device, time, slots, width, writes, reads, mixed, planted):
+    """``mixed``: every third token has a route to every row."""
+
+    print(f"recurrence T={time} N={slots} W={writes} mixed={mixed} {planted}", flush=True)
+    a = _case(time, slots, width, writes, reads, seed=time + slots)
+
+    def inputs():
+        routes = {}
+        for k in ("write", "read"):
+            x = serial.dense_routes(a[f"{k}_indices"][None], a[f"{k}_weights"][None],
+                                    slots).astype(np.float32)
+            if mixed:
+                x[:, 1:-1:3] += np.float32(0.2 / slots)
+            routes[f"{k}_routes"] = x
+        return dict(initial_memory=a["m0"][None], values=a["values"][None],
+                    input_gate=a["input_gate"][None], erase_gate=a["input_gate"][None],
+                    forget_log_gate=a["forget_log_gate"][None], **routes)
+
+    def run(x):
+        return cow.sdm_recurrence(**{k: torch.from_numpy(v.copy()).to(device)
+                                     for k, v in x.items()}, return_states=True)
+
+    before = run(inputs())
+    t = _plant(a, planted)
+    if mixed and planted == "overflow":
+        # the row's 3e38 would reach the others through the tokens of all rows
+        a["m0"][a["write_indices"][t, 0], COLUMN] = 0.0
+        a["values"][t, COLUMN] = np.inf
+    x = inputs()
+    if mixed and "last overflow" in planted:
+        row = a["write_indices"][t, 0]
+        x["write_routes"][:, :t, row] = x["read_routes"][:, :t, row] = 0.0
+    readings, final, states = run(x)
+    want = _dense_sums(x["initial_memory"], x["write_routes"], x["values"], x["input_gate"],
+                       x["forget_log_gate"], x["read_routes"], x["erase_gate"])
+    for got, expected in zip((readings, final, states), want):
+        _assert_same(got, expected)
+    r2, m2 = cow.sdm_recurrence(**{k: torch.from_numpy(v.copy()).to(device)
+                                   for k, v in x.items()})
+    assert torch.equal(r2.nan_to_num(1.5), readings.nan_to_num(1.5))
+    assert torch.equal(m2.nan_to_num(1.5), final.nan_to_num(1.5))
+    if "overflow" not in planted:
+        assert torch.equal(readings[:, :t], before[0][:, :t])
+        assert torch.equal(states[:, :t], before[2][:, :t])
+    if "memory" in planted or "value" in planted:
+        others = [c for c in range(width) if c != COLUMN]
+        for got, same in zip((readings, final, states), before):
+            assert torch.equal(got[..., others], same[..., others])
