@@ -14,21 +14,23 @@
 // zero.  Producer waves compact every vector to its nonzero entries while the
 // tokens before it run, and the recurrence then touches only those rows, as
 // in route_recurrence.hip (the table of 32 columns in LDS, 8 lanes to a
-// column, the same pipeline).  A vector with more than 8 nonzero write or 32
-// nonzero read routes makes its token a dense one: every row, lane g of a
-// column the rows g, g + 8, ....  A token's arithmetic depends on its own
-// vectors only, so later tokens never change earlier results.
+// column, the same pipeline).  A token with more than 8 nonzero write or 32
+// nonzero read routes is a dense one, and from its first dense token on a
+// sequence is left to a kernel that holds the memory in registers and sums
+// over every row (below), launched behind this one: it goes on from the memory
+// that this one leaves before that token.  A token's arithmetic depends on the
+// vectors up to its own, so later tokens never change earlier results.
 //
 // A zero route times a row, or a delta, that is not finite is NaN in the dense
 // sums.  Every lane starts its sums from 0 * the rows it wrote, so a column
 // that met one reads NaN from that token to the last; at the end its wave
-// takes it again with every token a dense one, and stores what follows the
-// first reading that is not finite.
+// takes it again with sums over every row, and stores what follows the first
+// reading that is not finite.
 //
-// A dense token costs 5.7 us here (N = 256) and 0.8 us with the memory in
-// registers, so a sequence whose first token is dense is left to a kernel
-// that holds it so (below): both are launched, and each takes its sequences.
-// The first token alone decides, which keeps a prefix's results its own.
+// A dense token costs 0.8 us there (N = 256) and 3.9 here with every row in
+// LDS, so one is enough to hand a sequence over: 128 tokens of 16 writes behind
+// a first token without any, B = 16, D = 128, 506 -> 114 us, 715 -> 287 with the
+// per-token memories.
 //
 // Per-token memories (the backward's input) are 4 N D bytes a token, written
 // by four waves of their own from LDS, 16 bytes a lane and a table row's 32
@@ -74,14 +76,14 @@ struct RecParams {
   const float* eg;       // [B, T]
   const float* flg;      // [B, T]
   const float* rr;       // [B, T, N]
+  int64_t* stops;        // [B]: a sequence's first dense token, T without one
   float* readings;       // [B, T, D]
   float* states;         // [B, T, N, D] or null
   float* final_memory;   // [B, N, D] or null
 };
 
-// Whether a sequence is one of sparse tokens, by its first token's vectors
-// (the same in every wave that asks).
-__device__ __forceinline__ bool sparse_sequence(const float* w, const float* r, int N) {
+// Whether a token is not a dense one (the same in every wave that asks).
+__device__ __forceinline__ bool sparse_token(const float* w, const float* r, int N) {
   const int lane = static_cast<int>(threadIdx.x) % kWave;
   int writes = 0, reads = 0;
 #pragma unroll 4
@@ -100,13 +102,15 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// A wave's columns that are `bad` (the same in a column's lanes), from the
-// initial memory on with every token a dense one: the table (`mine`: the
-// column's) is left as the final memory, and readings and per-token memories
-// are stored from the first reading that is not finite.
+// A wave's columns that are `bad` (the same in a column's lanes), `end` tokens
+// from the initial memory on with sums over every row: the table (`mine`: the
+// column's) is left as the memory behind them (before token T and without
+// per-token memories it also goes to where the next kernel looks for it), and
+// readings and per-token memories are stored from the first reading that is
+// not finite.
 template <bool STATES>
 __device__ __forceinline__ void redo_columns(const RecParams& P, char* mine, int64_t b, int d,
-                                             int g, bool bad) {
+                                             int g, int64_t end, bool bad) {
   const int N = P.slots, D = P.width;
   const int64_t T = P.time;
   float* const readings = P.readings + b * T * D + (bad ? d : 0);
@@ -115,7 +119,7 @@ __device__ __forceinline__ void redo_columns(const RecParams& P, char* mine, int
     return reinterpret_cast<float*>(mine + n * kRrRowBytes);
   };
   __threadfence();   // the wave's own readings, by other lanes of it
-  int64_t from = T;
+  int64_t from = end;
   for (int64_t t = g; bad && t < from; t += kRrGroups) {
     if (!finite(readings[t * D])) from = t;
   }
@@ -127,7 +131,7 @@ __device__ __forceinline__ void redo_columns(const RecParams& P, char* mine, int
   for (int n = g; n < N; n += kRrGroups) {
     if (bad) *row(n) = P.m0[(b * N + n) * static_cast<int64_t>(D) + d];
   }
-  for (int64_t t = 0; t < T; ++t) {
+  for (int64_t t = 0; t < end; ++t) {
     const int64_t bt = b * T + t;
     const float* const wt = P.wr + bt * N;
     const float* const rt = P.rr + bt * N;
@@ -161,6 +165,11 @@ __device__ __forceinline__ void redo_columns(const RecParams& P, char* mine, int
     // readings are already
     if (!STATES && __ballot(bad && delta == delta) == 0) break;
   }
+  if (!STATES && end < T) {
+    for (int n = g; n < N; n += kRrGroups) {
+      if (bad) P.final_memory[(b * N + n) * static_cast<int64_t>(D) + d] = *row(n);
+    }
+  }
 }
 
 // V: floats per access to the memories, 4 when D % 4 == 0 and they are
@@ -179,9 +188,12 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
   const int cols = nw * kRrCols;
   const int N = P.slots, D = P.width, CH = kDrChunk;
   const int64_t T = P.time;
-  // the whole workgroup again: every wave counts the same vectors
-  if (T > 0 && !sparse_sequence(P.wr + b * T * N, P.rr + b * T * N, N)) return;
   const int tid = static_cast<int>(threadIdx.x);
+  // the whole workgroup again: every wave counts the same vectors
+  if (T > 0 && !sparse_token(P.wr + b * T * N, P.rr + b * T * N, N)) {
+    if (block == 0 && tid == 0) P.stops[b] = 0;
+    return;
+  }
   const int lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int table_bytes = (N + 1) * kRrRowBytes;   // a wave's table, row N unused by routes
@@ -196,9 +208,16 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
                                   (c % kRrCols) * 4);
   };
   // 0 or NaN per column: whether the initial memory holds a non-finite value
-  int* const redo = reinterpret_cast<int*>(poison + cols);   // set: some columns are taken again
+  // the sequence's first dense token, set by the compute waves in its chunk
+  // (all the same value), for all others at the end of that chunk; whether
+  // some columns are taken again
+  int64_t* const stop = reinterpret_cast<int64_t*>(poison + cols);
+  int* const redo = reinterpret_cast<int*>(stop + 1);
   if (tid < cols) poison[tid] = 0.0f;
-  if (tid == 0) *redo = 0;
+  if (tid == 0) {
+    *stop = INT64_MAX;
+    *redo = 0;
+  }
   __syncthreads();
   {
     const float* const m0 = P.m0 + b * N * static_cast<int64_t>(D);
@@ -229,6 +248,15 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
   const int64_t chunks = (T + CH - 1) >> kDrShift;
   const int col = lane / kRrGroups, g = lane % kRrGroups;
   float pz = 0.0f;   // compute waves: NaN once a row was not finite
+  // Whether the sequence ends in chunk c.  A wave asks after the chunk's last
+  // barrier, and what a faster one may have set by then is a later chunk's.
+  // (A relaxed load: a volatile one waits for the wave's stores.  Once a chunk:
+  // asked for every token by the store waves it took 10 us of 100 at B = 16,
+  // T = 128, N = 256, D = 128.)
+  auto stops_in = [&](int64_t c) __attribute__((always_inline)) {
+    return (__hip_atomic_load(stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >> kDrShift) <=
+           c;
+  };
   if (wave >= nw && wave < nw + kDrProducers / kWave) {
     // ---- producers: wave pw takes the tokens pw, pw + 8, ..., kAhead of them
     // loaded before they are needed.  A token is compacted in parts, one
@@ -340,6 +368,7 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
         if (c < chunks) chunk(c, false);
         __syncthreads();
       }
+      if (stops_in(c - 1)) break;
     }
   } else if (STATES && wave >= nw) {
     // ---- the per-token memories: the table as it is between a token's barriers
@@ -352,23 +381,28 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
     float* out = P.states + (b * T * N + n0) * static_cast<int64_t>(D) + d0 + cc;
     __syncthreads();
     // (every lane takes part in the barriers, so the loops are the same in all)
-    for (int64_t t = 0; t < chunks << kDrShift; ++t, out += static_cast<int64_t>(N) * D) {
-      lds_barrier();
-      float* to = out;
-      for (int first = 0; first < N; first += rows) {
-        Copy v[kDrCopy];
+    for (int64_t c = 0; c < chunks; ++c) {
+      const int64_t left = T - (c << kDrShift);
+      const int in = static_cast<int>(left < CH ? left : CH);   // tokens of the chunk
+      for (int j = 0; j < CH; ++j, out += static_cast<int64_t>(N) * D) {
+        lds_barrier();
+        float* to = out;
+        for (int first = 0; first < N; first += rows) {
+          Copy v[kDrCopy];
 #pragma unroll
-        for (int q = 0; q < kDrCopy; ++q) {
-          const int n = first + n0 + q * copiers;
-          v[q] = *reinterpret_cast<const Copy*>(table_at(n < N ? n : N, cc));
-        }
-        if (first + rows >= N) lds_barrier();   // the last rows are in registers
+          for (int q = 0; q < kDrCopy; ++q) {
+            const int n = first + n0 + q * copiers;
+            v[q] = *reinterpret_cast<const Copy*>(table_at(n < N ? n : N, cc));
+          }
+          if (first + rows >= N) lds_barrier();   // the last rows are in registers
 #pragma unroll
-        for (int q = 0; q < kDrCopy; ++q) {
-          if (on && t < T && first + n0 + q * copiers < N) *reinterpret_cast<Copy*>(to) = v[q];
-          to += static_cast<int64_t>(copiers) * D;
+          for (int q = 0; q < kDrCopy; ++q) {
+            if (on && j < in && first + n0 + q * copiers < N) *reinterpret_cast<Copy*>(to) = v[q];
+            to += static_cast<int64_t>(copiers) * D;
+          }
         }
       }
+      if (stops_in(c)) break;
     }
   } else {
     // ---- compute waves
@@ -376,6 +410,8 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
     char* const mine = lds + wave * table_bytes + col * 4;   // this column's table
     const int d = d0 + wave * kRrCols + col;
     pz = poison[wave * kRrCols + col];
+    bool stopped = false;   // at a dense token, with pz before it
+    float pz_before = 0.0f;
     // a token's two barriers: its update is done; its memory has been read out
     auto updated = [&]() __attribute__((always_inline)) { if (STATES) lds_barrier(); };
     auto copied = [&]() __attribute__((always_inline)) { if (STATES) lds_barrier(); };
@@ -475,67 +511,55 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
             __builtin_amdgcn_sched_barrier(0);
           }
         } else {
-          // one token after the other: the sparse ones in the arithmetic
-          // above, the dense ones over all rows
+          // one token after the other, in the arithmetic above, up to the
+          // first dense one; what follows only keeps the barriers, and its
+          // results are the next kernel's
           const float before = last_reading();
           keep = g == kRrGroups - 1 ? before : keep;
           if (j0 > 0 && t < T && d < D) *out = keep;
-          float reading = 0.0f;
-          for (int u = 0; u < kRrGroups; ++u) {
-            const char* const rec = pw + u * Rec::kBytes;
+          const int first = stopped ? 0 : __builtin_ctz(dense);
+          for (int u = 0; u < first; ++u) {
+            const uint2 e = entry(pw + u * Rec::kBytes);
             gates = *reinterpret_cast<const float4*>(pg + u * Rec::kBytes);
             gv = gates.y * *reinterpret_cast<const float*>(pv + u * Rec::kBytes);
-            float sum;
-            if ((dense >> u) & 1u) {
-              const int64_t token = (b * T + (c << kDrShift) + j0 + u) * N;
-              const float* const wt = P.wr + token;
-              const float* const rt = P.rr + token;
-              float part = 0.0f;
-#pragma unroll 8
-              for (int n = g; n < N; n += kRrGroups) {
-                const float w = wt[n];
-                const float m = *at_row(n * kRrRowBytes);
-                part = __builtin_fmaf(w, w != 0.0f ? m * gates.x : m, part);
-              }
-              const float delta = __builtin_fmaf(-gates.z, column_sum8(part), gv);
-              sum = 0.0f;
-#pragma unroll 8
-              for (int n = g; n < N; n += kRrGroups) {
-                const float w = wt[n];
-                float* const p = at_row(n * kRrRowBytes);
-                const float m = *p;
-                const float now = __builtin_fmaf(w, delta, w != 0.0f ? m * gates.x : m);
-                *p = now;
-                pz = __builtin_fmaf(now, 0.0f, pz);
-                sum = __builtin_fmaf(rt[n], now, sum);
-              }
-              updated();
-            } else {
-              const uint2 e = entry(rec);
-              float* const p = at_row(e.x);
-              const float w = __uint_as_float(e.y);
-              const float m = *p * (w != 0.0f ? gates.x : 1.0f);
-              const float delta = __builtin_fmaf(-gates.z,
-                                                 column_sum8(__builtin_fmaf(w, m, pz)), gv);
-              const float now = __builtin_fmaf(w, delta, m);
-              *p = now;
-              pz = __builtin_fmaf(now, 0.0f, pz);
-              updated();
-              sum = pz;
+            float* const p = at_row(e.x);
+            const float w = __uint_as_float(e.y);
+            const float m = *p * (w != 0.0f ? gates.x : 1.0f);
+            const float delta = __builtin_fmaf(-gates.z, column_sum8(__builtin_fmaf(w, m, pz)),
+                                               gv);
+            const float now = __builtin_fmaf(w, delta, m);
+            *p = now;
+            pz = __builtin_fmaf(now, 0.0f, pz);
+            updated();
+            float sum = pz;
 #pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                const uint2 q = entry(pr + u * Rec::kBytes + 8 * kRrGroups * i);
-                sum = __builtin_fmaf(__uint_as_float(q.y), *at_row(q.x), sum);
-              }
+            for (int i = 0; i < 4; ++i) {
+              const uint2 q = entry(pr + u * Rec::kBytes + 8 * kRrGroups * i);
+              sum = __builtin_fmaf(__uint_as_float(q.y), *at_row(q.x), sum);
             }
-            reading = column_sum8(sum);
+            const float reading = column_sum8(sum);
             keep = g == u ? reading : keep;
             copied();
           }
-          // the pipeline again from the next group's first token on; the
-          // last reading is summed once more there, as itself
+          if (!stopped) {
+            stopped = true;
+            pz_before = pz;
+            if (lane == 0) *stop = (c << kDrShift) + j0 + first;
+            if (!STATES && d < D && column_sum8(pz) == 0.0f) {   // others: redo_columns
+              // the memory before the dense token, where the next kernel
+              // looks for it (else it is the last per-token memory)
+              for (int n = g; n < N; n += kRrGroups) {
+                P.final_memory[(b * N + n) * static_cast<int64_t>(D) + d] =
+                    *at_row(n * kRrRowBytes);
+              }
+            }
+          }
+          for (int u = first; u < kRrGroups; ++u) {
+            updated();
+            copied();
+          }
           begin(kRrGroups);
-          old_pz = g == 0 ? reading : 0.0f;
+          old_pz = 0.0f;
         }
         pw += kRrGroups * Rec::kBytes;
         pr += kRrGroups * Rec::kBytes;
@@ -549,20 +573,25 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
       keep = g == kRrGroups - 1 ? reading : keep;
       if (t < T && d < D) *out = keep;
       if (!STATES) __syncthreads();
+      if (stopped) break;
     }
+    if (stopped) pz = pz_before;
   }
   // a column that was never other than finite keeps pz 0
   const bool bad = wave < nw && T > 0 && d0 + wave * kRrCols + col < D &&
                    !(column_sum8(pz) == 0.0f);
   if (bad) *redo = 1;
   __syncthreads();   // what the store waves wrote is out, too
+  const int64_t end = *stop < T ? *stop : T;
+  if (block == 0 && tid == 0 && T > 0) P.stops[b] = end;
   if (*redo) {
     if (__ballot(bad)) {
       redo_columns<STATES>(P, lds + wave * table_bytes + col * 4, b, d0 + wave * kRrCols + col, g,
-                           bad);
+                           end, bad);
     }
     __syncthreads();
   }
+  if (end < T) return;
   if (!P.final_memory) return;
   float* const out = P.final_memory + b * N * static_cast<int64_t>(D);
   const int at_once = static_cast<int>(blockDim.x) / per_row;
@@ -574,7 +603,7 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
   }
 }
 
-// ---- sequences of dense tokens
+// ---- sequences from their first dense token on
 //
 // A wave owns 4 columns of one batch row's memory for the whole sequence,
 // in registers: lane = 16 * column + row group, and row group g holds rows
@@ -675,11 +704,13 @@ __global__ __launch_bounds__(kRecThreads) void dense_recurrence_kernel(RecParams
   const int col = lane / kRecGroups;
   const int g = lane % kRecGroups;
   const int N = P.slots, D = P.width;
-  const int64_t T = P.time;
+  const int64_t start = P.all_dense ? 0 : P.stops[b];
+  const int64_t T = P.time - start;
+  if (!P.all_dense && T <= 0) return;
+  const int64_t first = b * P.time + start;   // of the tokens, over the batch
   const int d = cb * kRecCols + col;
   const bool col_ok = d < D;
   const int n0 = g * RPL;
-  if (!P.all_dense && sparse_sequence(P.wr + b * T * N, P.rr + b * T * N, N)) return;
 
   // the lane's rows in a [N, D] block: offset n0 * D + d, stride D (the
   // host keeps N * D below 2^31)
@@ -687,7 +718,10 @@ __global__ __launch_bounds__(kRecThreads) void dense_recurrence_kernel(RecParams
                        static_cast<uint32_t>(col_ok ? d : 0);
   float m[RPL];
   {
-    const float* src = P.m0 + b * N * static_cast<int64_t>(D);
+    // the memory before token `start` (recurrence_kernel's)
+    const float* src = start == 0 ? P.m0 + b * N * static_cast<int64_t>(D)
+                       : P.states ? P.states + (first - 1) * N * static_cast<int64_t>(D)
+                                  : P.final_memory + b * N * static_cast<int64_t>(D);
 #pragma unroll
     for (int i = 0; i < RPL; ++i) {
       const bool in = col_ok && n0 + i < N;
@@ -695,8 +729,8 @@ __global__ __launch_bounds__(kRecThreads) void dense_recurrence_kernel(RecParams
       m[i] = in ? v : 0.0f;
     }
   }
-  const float* const wr_b = P.wr + b * T * N;
-  const float* const rr_b = P.rr + b * T * N;
+  const float* const wr_b = P.wr + first * N;
+  const float* const rr_b = P.rr + first * N;
   // ring of PF tokens' route vectors and values: slot j holds token t0 + j
   // of the current round, and is refilled with token t + PF as soon as
   // token t is done.  Every load is a vector load, so a wait for the oldest
@@ -706,13 +740,13 @@ __global__ __launch_bounds__(kRecThreads) void dense_recurrence_kernel(RecParams
     load_rows<RPL, V4>(wr_b + t * N, n0, N, w[j]);
     load_rows<RPL, V4>(rr_b + t * N, n0, N, r[j]);
     // a lane past the width computes on column 0's values and stores nothing
-    val[j] = P.values[(b * T + t) * D + (col_ok ? d : 0)];
+    val[j] = P.values[(first + t) * D + (col_ok ? d : 0)];
   };
   // the gates of 64 tokens, lane k holding token 64c + k's, a chunk ahead
   float gates[2][3];
   auto fetch_gates = [&](int slot, int64_t c) __attribute__((always_inline)) {
     const int64_t t = c * kWave + lane;
-    const int64_t bt = b * T + (t < T ? t : 0);
+    const int64_t bt = first + (t < T ? t : 0);
     gates[slot][0] = P.flg[bt];
     gates[slot][1] = P.ig[bt];
     gates[slot][2] = P.eg[bt];
@@ -728,7 +762,7 @@ __global__ __launch_bounds__(kRecThreads) void dense_recurrence_kernel(RecParams
     for (int j = 0; j < PF; ++j) {
       const int64_t t = t0 + j;
       if (t >= T) break;
-      const int64_t bt = b * T + t;
+      const int64_t bt = first + t;
       const int k = static_cast<int>(t % kWave);
       const int slot = static_cast<int>((t / kWave) & 1);
       float fg, in_g, er_g;
@@ -764,6 +798,7 @@ __global__ __launch_bounds__(kRecThreads) void dense_recurrence_kernel(RecParams
 #pragma unroll
       for (int i = 0; i < RPL; ++i) {
         m[i] = __builtin_fmaf(wj[i], delta, m[i]);
+        if (!EXACT && n0 + i >= N) m[i] = 0.0f;   // 0 * a delta that is not finite
         rp = __builtin_fmaf(rj[i], m[i], rp);
       }
       // the slot takes token t + PF (the last token again near the end, so
@@ -859,7 +894,7 @@ template <int V, int SEG, bool STATES>
 int32_t launch_recurrence(RecParams& P, hipStream_t s) {
   auto bytes = [&](int nw) {
     return nw * (P.slots + 1) * kRrRowBytes + 2 * (kDrChunk + kRrPad) * RrRecord<1, 4>::kBytes +
-           4 * nw * kRrCols + 4;
+           4 * nw * kRrCols + 16;
   };
   // the waves that D fills, fewer where the tables and the stage would not
   // fit in LDS
@@ -897,6 +932,11 @@ int32_t launch_recurrence_slots(RecParams& P, hipStream_t s) {
 using namespace cowsdm_impl;
 
 extern "C" int32_t cowsdm_recurrence_forward(const cowsdm_recurrence_t* r, void* stream) {
+  return cowsdm_recurrence_forward_stops(r, nullptr, stream);
+}
+
+extern "C" int32_t cowsdm_recurrence_forward_stops(const cowsdm_recurrence_t* r, int64_t* stops,
+                                                   void* stream) {
   if (!r) return fail(COWSDM_EARG, "recurrence: null argument");
   if (r->batch < 0 || r->time < 0 || r->slots <= 0 || r->width <= 0) {
     return fail(COWSDM_EARG, "recurrence: invalid sizes");
@@ -927,6 +967,7 @@ extern "C" int32_t cowsdm_recurrence_forward(const cowsdm_recurrence_t* r, void*
   P.eg = r->erase_gate;
   P.flg = r->forget_log_gate;
   P.rr = r->read_routes;
+  P.stops = stops;
   P.readings = r->readings;
   P.states = r->states;
   P.final_memory = r->final_memory;
@@ -941,16 +982,20 @@ extern "C" int32_t cowsdm_recurrence_forward(const cowsdm_recurrence_t* r, void*
   // with B = 64, D = 128); without them it is not (52 us against 30), but both
   // calls have to give the same readings.  And the sparse sequences' launch, at
   // most 16 waves to 16 columns, has to stay below 2^32 threads.
-  P.all_dense = (P.slots <= kWave && P.batch * P.width < 4096) ||
+  // Without a place for where sequences are handed over, and for their memory
+  // there, none is.
+  P.all_dense = !P.stops || (!P.states && !P.final_memory) ||
+                (P.slots <= kWave && P.batch * P.width < 4096) ||
                 (P.batch + kXcds - 1) * ((P.width + 15) / 16) >= (int64_t{1} << 22);
-  if (P.time > 0 || P.all_dense) {
-    const int32_t rc = launch_dense_sequences(P, s);
-    if (rc || P.all_dense) return rc;
-  }
-  if (P.states) {
-    return v4 ? launch_recurrence_slots<4, true>(P, s) : launch_recurrence_slots<1, true>(P, s);
-  }
-  return v4 ? launch_recurrence_slots<4, false>(P, s) : launch_recurrence_slots<1, false>(P, s);
+  if (P.all_dense) return launch_dense_sequences(P, s);
+  RecParams sparse = P;
+  const int32_t rc =
+      P.states ? (v4 ? launch_recurrence_slots<4, true>(sparse, s)
+                     : launch_recurrence_slots<1, true>(sparse, s))
+               : (v4 ? launch_recurrence_slots<4, false>(sparse, s)
+                     : launch_recurrence_slots<1, false>(sparse, s));
+  // behind it, from each sequence's first dense token on
+  return rc || P.time == 0 ? rc : launch_dense_sequences(P, s);
 }
 
 extern "C" int32_t cowsdm_dense_routes(const float* weights, const void* indices,

@@ -92,6 +92,35 @@ def test_a_token_depends_on_its_own_vectors_only(device, mixed):
     assert torch.equal(s2[:, :t0], states[:, :t0])
 
 
+@pytest.mark.parametrize("slots,width", [(70, 130), (300, 12)])
+@pytest.mark.parametrize("first", [0, 1, 6, 7, 8, 15, 16, 31, 39])
+def test_hand_over_at_the_first_dense_token(device, first, slots, width):
+    """Sparse tokens, none with a route at first, up to token ``first`` and
+    dense ones from there on: the oracle's results, and what comes before is
+    the shorter sequence's, bit for bit."""
+
+    print(f"hand over at {first} N={slots} D={width}", flush=True)
+    a = _inputs(3, 40, slots, width, seed=first, mixed=False)
+    a["write_routes"][:, 0] = a["read_routes"][:, 0] = 0.0
+    rng = np.random.default_rng(first)
+    a["write_routes"][1:, first] = _routes(rng, np.array([9, slots]), slots)
+    a["write_routes"][0, first:] = _routes(rng, np.full(40 - first, 16), slots)
+    a["read_routes"][0, first] = 0.0
+    g = _gpu(a, device)
+    readings, final, states = cow.sdm_recurrence(**g, return_states=True)
+    scale = min(16.0, slots / 4)
+    for got, want in zip((readings, final, states), _oracle(a)):
+        np.testing.assert_allclose(got.cpu().numpy(), want, rtol=scale * RTOL, atol=scale * ATOL)
+    assert torch.equal(states[:, -1], final)
+    r2, m2 = cow.sdm_recurrence(**g)
+    assert torch.equal(r2, readings) and torch.equal(m2, final)
+    if first:
+        part = {k: (v[:, :first].contiguous() if k != "initial_memory" else v)
+                for k, v in g.items()}
+        r0, m0 = cow.sdm_recurrence(**part)
+        assert torch.equal(r0, readings[:, :first]) and torch.equal(m0, states[:, first - 1])
+
+
 @pytest.mark.parametrize("mixed", [False, True])
 @pytest.mark.parametrize("planted", ["memory", "value", "weight", "read"])
 def test_not_finite(device, mixed, planted):
