@@ -411,12 +411,16 @@ def lib() -> ctypes.CDLL:
                     "copy-on-write SDM kernels have no CPU fallback"
                 )
             handle = ctypes.CDLL(str(path), mode=ctypes.RTLD_LOCAL)
-            for name, (restype, argtypes) in SIGNATURES.items():
-                fn = getattr(handle, name)
-                fn.restype = restype
-                fn.argtypes = argtypes
             if handle.cowsdm_abi_version() != ABI_VERSION:
                 raise RuntimeError("libcowsdm.so ABI version mismatch")
+            for name, (restype, argtypes) in SIGNATURES.items():
+                # entries are added within a version: an older build lacks some
+                fn = getattr(handle, name, None)
+                if fn is None:
+                    raise RuntimeError(f"{path} has no {name}: it is older than this package, "
+                                       "build it again")
+                fn.restype = restype
+                fn.argtypes = argtypes
             _lib = handle
     return _lib
 
