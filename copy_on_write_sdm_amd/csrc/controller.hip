@@ -3,11 +3,12 @@
 // LayerNorm, the read / write key, value, forget and input projections and
 // the gates; after it, the readings LayerNorm, the sigmoid output gate and
 // the output projection.  Routes are selected from the keys by
-// cowsdm_product_key_routes (routes.hip), or, for sqrt(N) <= 64, by the
-// prepare kernel itself once its tokens' keys are out (one wave per route
-// row, routes.h): cowsdm_controller_prepare_routes; with nothing between two
-// layers, one layer's finish and the next one's prepare and routes share a
-// launch (cowsdm_controller_finish_prepare_routes).
+// cowsdm_product_key_routes (routes.hip), or, where that is faster
+// (prepare_selects), by the prepare kernel itself once its tokens' keys are
+// out (one wave per route row, routes.h): cowsdm_controller_prepare_routes;
+// with nothing between two layers, one layer's finish and the next one's
+// prepare and routes then share a launch too
+// (cowsdm_controller_finish_prepare_routes).
 //
 // The projections are products [tokens, width] x [width, rows] in float32 on
 // the matrix cores (v_mfma_f32_16x16x4_f32): a wave computes tiles of 16 MT
@@ -741,9 +742,8 @@ int32_t prepare_params(const cowsdm_controller_t* c, const float* tokens, int64_
 template <int MR, int MW>
 int32_t launch_prepare_routes(CtlParams P, const CtlRoutes& R, hipStream_t s) {
   P.tokens_per_group = few_tokens(P.batch);
-  const size_t lds = token_lds(P, 1);
+  const size_t lds = token_lds(P, 1);   // at most 256 inputs a token (prepare_selects)
   auto* const kernel = &controller_prepare_routes_kernel<MR, MW>;
-  if (int32_t e = allow_lds(reinterpret_cast<const void*>(kernel), lds)) return e;
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(token_groups(P))), dim3(kCtlThreads),
                      lds, s, P, R);
   return launch_status("controller prepare routes");
@@ -755,7 +755,6 @@ int32_t launch_finish_prepare_routes(CtlParams F, CtlParams P, const CtlRoutes& 
   F.tokens_per_group = P.tokens_per_group = few_tokens(P.batch);
   const size_t lds = token_lds(P, 2);
   auto* const kernel = &controller_finish_prepare_routes_kernel<MR, MW>;
-  if (int32_t e = allow_lds(reinterpret_cast<const void*>(kernel), lds)) return e;
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(token_groups(P))), dim3(kCtlThreads),
                      lds, s, F, P, R, kCtlMaxWaves / 2);
   return launch_status("controller finish and prepare");
@@ -814,6 +813,28 @@ int32_t by_tokens(const CtlParams& P, int lds_rows, One one, Two two, Many many)
 // How a wave selects its rows' routes (controller_route_row's M).
 int route_m(const CtlRoutes& R, int sub, int k) {
   return route_row_sorted(R.root, k) ? 0 : route_pair_m(sub, k);
+}
+
+// Whether a prepare selects its routes itself, in workgroups of 16 waves that
+// project every row of their tokens: `rows` route rows (of a read or write
+// route each) and P's projection.  Its row tiles then take a round of the
+// waves each 16, and a round about as long as its chunks of 128 inputs, where
+// the separate prepare shares the tiles out to more workgroups.  The two more
+// launches take 4 us where the kernels are short and 6 us of the host
+// (prepare_sdm_step 22 us against 28), so the line lies where the fused kernel
+// passes that.  16 tokens, rounds x chunks: 1 (width 128, N = 256, 1 head)
+// 8.7 us against 13.0, 3 (4 heads of N = 1,024) 14.0 against 12.6, 4 (width
+// 256, 2 heads) 16.8 against 13.3, 5 (width 128, 8 heads of N = 1,024) 20
+// against 12.5, 8 (width 256, 4 heads of N = 1,024) 26 against 14, 16 (width
+// 400, 4 heads of N = 1,024) 45 against 16, 72 (width 1,024, 8 heads) 218
+// against 21.  And from more tokens than one workgroup of 16 each on every
+// compute unit on, a second one waits: 4,096 rows of 1 head 15.8 against 17.5,
+// 6,000 28 against 20; of 4 heads 17.9 against 17.4, 22.9 against 20.6 at 8,192.
+bool prepare_selects(const CtlParams& P, int root, int64_t rows) {
+  const int rounds = (P.rows + kCtlTile * kCtlMaxWaves - 1) / (kCtlTile * kCtlMaxWaves);
+  const int chunk = kCtlGroup * ctl_chunk<1, 1>();
+  return root <= kWave && rounds * ((P.width + chunk - 1) / chunk) <= 5 &&
+         rows <= kCtlTile * kCtlUnits;
 }
 
 // The route geometry of `reads` and `writes` selections over c's slots and
@@ -894,9 +915,7 @@ extern "C" int32_t cowsdm_controller_prepare_routes(
   }
   if (batch == 0) return 0;
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  if (R.root > kWave || batch * c->heads >= kRouteLaneRows) {
-    // a shortlist of more than one entry per lane, or rows enough for a lane
-    // each: the separate launches
+  if (!prepare_selects(P, R.root, batch * c->heads)) {
     if (int32_t e = cowsdm_controller_prepare(c, tokens, batch, normalized, read_keys,
                                               write_keys, values, input_gate, forget_log_gate,
                                               stream)) {
@@ -969,8 +988,7 @@ extern "C" int32_t cowsdm_controller_finish_prepare_routes(
     return e;
   }
   if (batch == 0) return 0;
-  if (R.root > kWave || batch * c->heads >= kRouteLaneRows) {
-    // the next layer's routes take their own launches: finish, then prepare
+  if (!prepare_selects(P, R.root, batch * next->heads)) {
     if (int32_t e = cowsdm_controller_finish_residual(c, normalized, reading, batch, out,
                                                       residual, out_sum, stream)) {
       return e;

@@ -61,3 +61,38 @@ def test_tiles_match_oracle_and_any_batch(device, width, heads, slots, batch):
                  "write_indices", "write_weights"):
         assert torch.equal(getattr(again.inputs, name), getattr(inp, name)[banks]), name
     assert torch.equal(ctl.finish_sdm_step(c, again, reading[banks]), out[some])
+
+
+@pytest.mark.parametrize("width,heads,slots,reads,batch", [
+    (128, 1, 256, 16, 4096), (128, 1, 256, 16, 4097), (64, 4, 256, 24, 1024),
+    (64, 4, 256, 24, 1025), (128, 8, 1024, 16, 9), (272, 1, 256, 16, 9), (240, 1, 1024, 32, 9)])
+def test_both_sides_of_the_fused_selection(device, width, heads, slots, reads, batch):
+    """Routes selected in the prepare's launch and in their own (more than
+    4,096 rows, or more than five rounds of a chunk of inputs in the fused
+    kernel): the same bits, which are product_key_routes' of the keys."""
+
+    from copy_on_write_sdm_amd import _native as nat
+    from copy_on_write_sdm_amd.routing import product_key_routes
+
+    print(f"fused selection width={width} H={heads} N={slots} R={reads} B={batch}", flush=True)
+    layer = make_layer(width, slots=slots, reads=reads, writes=4, heads=heads, seed=batch,
+                       dtype=torch.float32)
+    c = ctl.SDMController.from_module(layer, device=device)
+    x = torch.randn(batch, 1, width, device=device)
+    inp = ctl.prepare_sdm_step(c, x).inputs
+    rows, key = batch * heads, c.key_width_per_head
+    f = lambda *shape: torch.empty(*shape, device=device)
+    normalized, read_keys, write_keys = f(batch, width), f(rows, 1, key), f(rows, 1, key)
+    values, gate, forget = f(rows, c.head_width), f(rows), f(rows)
+    nat.check(nat.lib().cowsdm_controller_prepare(
+        c.c_struct(), x.data_ptr(), batch, normalized.data_ptr(), read_keys.data_ptr(),
+        write_keys.data_ptr(), values.data_ptr(), gate.data_ptr(), forget.data_ptr(),
+        nat.stream_handle(device)), "prepare")
+    assert torch.equal(inp.values, values) and torch.equal(inp.forget_log_gate, forget)
+    for keys, k, name in ((read_keys, reads, "read"), (write_keys, 4, "write")):
+        weights, indices = product_key_routes(keys, slots=slots, selected=k)
+        assert torch.equal(getattr(inp, f"{name}_indices"), indices[:, 0])
+        assert torch.equal(getattr(inp, f"{name}_weights"), weights[:, 0])
+    alone = ctl.prepare_sdm_step(c, x[-1:]).inputs
+    assert torch.equal(alone.read_indices, inp.read_indices[-heads:])
+    assert torch.equal(alone.read_weights, inp.read_weights[-heads:])
