@@ -1420,15 +1420,17 @@ def packed_sdm_cow_step(
         first = torch.empty(banks, device=device, dtype=torch.int64)
         repeated = torch.empty(banks, device=device, dtype=torch.int64)
         allocated = torch.empty((), device=device, dtype=torch.int32)
-    if state.paged_map is not None and banks:
-        state.paged_map.prove(banks * writes)
     shape = _shape(banks, slots, width, writes, reads, state.shared_initial_memory.shape[0],
                    index_code)
     floats = (write_weights, values, input_gate, effective_erase, forget_log_gate, read_weights)
+    proven = state.paged_map is None or not banks
     while True:
         if not types:
             floats = tuple(_widen(t) for t in floats)
             _check_float_tensors(floats)
+        if not proven:
+            state.paged_map.prove(banks * writes)
+            proven = True
         write_weights, values, input_gate, effective_erase, forget_log_gate, read_weights = floats
         output = torch.empty_like(values)
         layer = _step_layer(state, None, write_indices, write_weights, values, input_gate,

@@ -58,3 +58,20 @@ def test_narrow_inputs_equal_widened_ones(device, banks, slots, width, writes, r
     assert torch.equal(states[0].logical_to_physical, states[1].logical_to_physical)
     for a, b in ((states[0].materialize_dense(), states[1].materialize_dense()), tables):
         assert torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_a_refused_step_takes_no_pages(device, name):
+    """Weights, values and gates that no step takes are refused before a paged
+    map is given room for the step."""
+
+    print(f"refused step, {name} in float64", flush=True)
+    m0, steps = make_case(banks=4, slots=64, width=32, writes=2, reads=4, steps=1, seed=1)
+    state = cow.PackedSDMCopyOnWriteState.allocate(m0.to(device), banks=4, capacity_rows=256,
+                                                   map_page_slots=16)
+    before = state.paged_map.pages_bound, state.paged_map.capacity
+    x = to_device(steps[0], device)
+    x[name] = x[name].double()
+    with pytest.raises(ValueError, match="float32 weights, values and gates"):
+        cow.packed_sdm_cow_step(state, **x)
+    assert (state.paged_map.pages_bound, state.paged_map.capacity) == before
