@@ -19,7 +19,10 @@
 // sequence is left to a kernel that holds the memory in registers and sums
 // over every row (below), launched behind this one: it goes on from the memory
 // that this one leaves before that token.  A token's arithmetic depends on the
-// vectors up to its own, so later tokens never change earlier results.
+// vectors up to its own, so later tokens never change earlier results.  (With
+// up to 64 slots it also depends on whether batch x width is below 4,096, see
+// the rule in cowsdm_recurrence_forward_stops: there a batch row's results
+// differ in rounding between a small batch and a large one.)
 //
 // A zero route times a row, or a delta, that is not finite is NaN in the dense
 // sums.  Every lane starts its sums from 0 * the rows it wrote, so a column
@@ -977,11 +980,13 @@ extern "C" int32_t cowsdm_recurrence_forward_stops(const cowsdm_recurrence_t* r,
   const bool v4 = P.width % 4 == 0 && align % 16 == 0;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   // up to 64 slots and few columns the memory in registers is the faster one
-  // with per-token memories (59 us against 82 at B = 1, T = 128, N = 32, 70
-  // against 82 at N = 64; 134 against 84 at N = 128, 104 against 89 at N = 32
-  // with B = 64, D = 128); without them it is not (52 us against 30), but both
-  // calls have to give the same readings.  And the sparse sequences' launch, at
-  // most 16 waves to 16 columns, has to stay below 2^32 threads.
+  // with per-token memories (T = 128, D = 64: 56 us against 74 at B = 1, N = 32,
+  // 70 against 75 at N = 64; with B = 64, D = 128 98 against 79 and 185 against
+  // 87); without them it is not (50 to 54 us against 27 to 30), but both calls
+  // have to give the same readings.  The line cannot lie at N or D alone: with
+  // either kernel for all of N <= 64 one of these sides loses a third or more.
+  // And the sparse sequences' launch, at most 16 waves to 16 columns, has to
+  // stay below 2^32 threads.
   // Without a place for where sequences are handed over, and for their memory
   // there, none is.
   P.all_dense = !P.stops || (!P.states && !P.final_memory) ||

@@ -92,6 +92,20 @@ def test_a_token_depends_on_its_own_vectors_only(device, mixed):
     assert torch.equal(s2[:, :t0], states[:, :t0])
 
 
+@pytest.mark.parametrize("slots,width", [(33, 64), (64, 130)])
+def test_batch_size_changes_rounding_only(device, slots, width):
+    """Up to 64 slots batch x width decides between two orders of summation:
+    the same rows on either side of 4,096 agree within the tolerance."""
+
+    print(f"batch sizes N={slots} D={width}", flush=True)
+    a = _gpu(_inputs(4096 // width + 1, 21, slots, width, seed=slots, mixed=False), device)
+    large = cow.sdm_recurrence(**a, return_states=True)
+    small = cow.sdm_recurrence(**{k: v[:3].contiguous() for k, v in a.items()},
+                               return_states=True)
+    for x, y in zip(small, large):
+        np.testing.assert_allclose(x.cpu().numpy(), y[:3].cpu().numpy(), rtol=RTOL, atol=ATOL)
+
+
 @pytest.mark.parametrize("slots,width", [(70, 130), (300, 12)])
 @pytest.mark.parametrize("first", [0, 1, 6, 7, 8, 15, 16, 31, 39])
 def test_hand_over_at_the_first_dense_token(device, first, slots, width):
