@@ -842,7 +842,7 @@ class PackedSDMCopyOnWriteState:
         """``append_banks_from`` for every layer of a stack: the live rows of
         all layers and the rows free for them are read once (three reads per
         layer before: 0.35 ms of the 0.8 ms that admitting 16 requests to 64
-        takes on 7 layers)."""
+        takes on 7 layers).  Layer by layer with a paged map among them."""
 
         if any(st.paged_map is not None or other.paged_map is not None
                for st, other in zip(states, others)):
@@ -945,7 +945,8 @@ class PackedSDMCopyOnWriteState:
     def retain_banks_layers(states: Sequence["PackedSDMCopyOnWriteState"],
                             bank_indices: Sequence[torch.Tensor]) -> None:
         """``retain_banks`` for every layer of a stack, its banks per layer,
-        with one read of all layers' checks (before any layer changes)."""
+        with one read of all layers' checks, before any layer changes (with
+        a paged map among them layer by layer, each checked on its own)."""
 
         if any(st.paged_map is not None for st in states):
             for st, banks in zip(states, bank_indices):
@@ -988,7 +989,8 @@ class PackedSDMCopyOnWriteState:
     def release_layers(states: Sequence["PackedSDMCopyOnWriteState"],
                        bank_indices: Sequence[torch.Tensor]) -> list[torch.Tensor]:
         """``release`` for every layer of a stack, its banks per layer, with
-        one read of all layers' checks (before any layer changes)."""
+        one read of all layers' checks, before any layer changes (with a
+        paged map among them layer by layer, each checked on its own)."""
 
         if any(st.paged_map is not None for st in states):
             released = []

@@ -2,7 +2,8 @@
 
 ``product_key_routes`` keeps the reference's name, arguments, return values
 and argument errors; the selection runs in ``cowsdm_product_key_routes``
-(csrc/routes.hip), one wave per route row.  The reference calls it twice per
+(csrc/routes.hip), one wave per route row or, for tables of up to 1,024 slots
+and many rows, one lane.  The reference calls it twice per
 decode step and layer, for the read and the write routes
 (inference.py:479-488), on ``[banks, 1, 2*sqrt(N)]`` projections.
 """
