@@ -324,7 +324,6 @@ SIGNATURES: dict[str, tuple] = {
         _I32, [ctypes.POINTER(Controller), _P, _P, _I64, _P, _P, _P, ctypes.POINTER(Controller),
                _P, _P, _P, _P, _P, _P, _I64, _I64, _P, _P, _P, _P, _P]),
     "cowsdm_recurrence_forward": (_I32, [ctypes.POINTER(Recurrence), _P]),
-    "cowsdm_recurrence_forward_stops": (_I32, [ctypes.POINTER(Recurrence), _P, _P]),
     "cowsdm_route_recurrence_forward": (_I32, [ctypes.POINTER(RouteRecurrence), _P]),
     "cowsdm_dense_routes": (_I32, [_P, _P, _I32, _I64, _I64, _I64, _P, _P, _P]),
     "cowsdm_host_report_alloc": (

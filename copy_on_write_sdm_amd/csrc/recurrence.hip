@@ -18,10 +18,11 @@
 // nonzero read routes is a dense one, and from its first dense token on a
 // sequence is left to a kernel that holds the memory in registers and sums
 // over every row (below), launched behind this one: it goes on from the memory
-// that this one leaves before that token.  A token's arithmetic depends on the
+// that this one leaves before that token, whose number it finds in the place of
+// the sequence's last reading (handed_over).  A token's arithmetic depends on the
 // vectors up to its own, so later tokens never change earlier results.  (With
 // up to 64 slots it also depends on whether batch x width is below 4,096, see
-// the rule in cowsdm_recurrence_forward_stops: there a batch row's results
+// the rule in cowsdm_recurrence_forward: there a batch row's results
 // differ in rounding between a small batch and a large one.)
 //
 // A zero route times a row, or a delta, that is not finite is NaN in the dense
@@ -32,7 +33,7 @@
 //
 // A dense token costs 0.8 us there (N = 256) and 3.9 here with every row in
 // LDS, so one is enough to hand a sequence over: 128 tokens of 16 writes behind
-// a first token without any, B = 16, D = 128, 506 -> 114 us, 715 -> 287 with the
+// a first token without any, B = 16, D = 128, 508 -> 114 us, 716 -> 291 with the
 // per-token memories.
 //
 // Per-token memories (the backward's input) are 4 N D bytes a token, written
@@ -40,16 +41,15 @@
 // columns (128 bytes) together, between two barriers of the token; the
 // compute waves load the next token's rows and sum the reading meanwhile.
 // (From the compute waves, each storing its 8 columns, 64 batch rows of 64
-// tokens took 210 us against 114: half-written 64-byte requests.)
+// tokens took 210 us against 112: half-written 64-byte requests.)
 //
 // Measured at T = 128, N = 256, D = 128, 4 writes, 16 reads, before (every
 // row of every token in registers) and after, time of the call: with the
-// per-token memories B = 16 275 -> 98 us (269 MB: 2.7 TB/s; what bounds it is
+// per-token memories B = 16 275 -> 88 us (269 MB: 3.1 TB/s; what bounds it is
 // the token's two barriers, 0.6 us a token, the bytes alone are 40 us), B = 64
-// and T = 64 338 -> 114 us (537 MB, 4.7 TB/s: the bytes); without them 101 ->
-// 35 us (the token's serial chain and the host's part of the call).  The
-// second launch, where it has nothing to do, costs 3-5 us, 20 at B = 64, N =
-// 1024, D = 256.
+// and T = 64 338 -> 112 us (537 MB, 4.8 TB/s: the bytes); without them 101 ->
+// 30 us (the token's serial chain and the host's part of the call).  The
+// second launch, where it has nothing to do, takes 4.7 us of them at B = 16.
 
 #include <type_traits>
 
@@ -79,11 +79,31 @@ struct RecParams {
   const float* eg;       // [B, T]
   const float* flg;      // [B, T]
   const float* rr;       // [B, T, N]
-  int64_t* stops;        // [B]: a sequence's first dense token, T without one
   float* readings;       // [B, T, D]
   float* states;         // [B, T, N, D] or null
   float* final_memory;   // [B, N, D] or null
 };
+
+// A sequence that is handed over at token `stop` holds these bits in the place
+// of its last token's reading, which is still to come, in every column: a NaN
+// that no sequence that is done leaves there (done_reading).
+constexpr uint32_t kDrNan = 0x7fc00000u;
+constexpr int64_t kDrMaxTime = int64_t{1} << 22;
+
+__device__ __forceinline__ float handed_over(int64_t stop) {
+  return __uint_as_float(kDrNan | static_cast<uint32_t>(stop + 1));   // stop + 1 < 2^22
+}
+
+__device__ __forceinline__ float done_reading(float x) {
+  return x != x ? __uint_as_float(kDrNan) : x;
+}
+
+// The token that the sequence of this last reading is handed over at, or -1.
+__device__ __forceinline__ int64_t handed_over_at(float last) {
+  const uint32_t bits = __float_as_uint(last);
+  return bits > kDrNan && bits < kDrNan + kDrMaxTime ? static_cast<int64_t>(bits - kDrNan) - 1
+                                                     : -1;
+}
 
 // Whether a token is not a dense one (the same in every wave that asks).
 __device__ __forceinline__ bool sparse_token(const float* w, const float* r, int N) {
@@ -157,7 +177,7 @@ __device__ __forceinline__ void redo_columns(const RecParams& P, char* mine, int
     }
     const float reading = column_sum8(sum);
     if (bad && t >= from) {
-      if (g == 0) readings[t * D] = reading;
+      if (g == 0) readings[t * D] = done_reading(reading);
       if (STATES) {
         for (int n = g; n < N; n += kRrGroups) {
           P.states[(bt * N + n) * static_cast<int64_t>(D) + d] = *row(n);
@@ -193,8 +213,9 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
   const int64_t T = P.time;
   const int tid = static_cast<int>(threadIdx.x);
   // the whole workgroup again: every wave counts the same vectors
+  float* const last_reading_out = P.readings + (b * T + T - 1) * D + block * cols + tid;
   if (T > 0 && !sparse_token(P.wr + b * T * N, P.rr + b * T * N, N)) {
-    if (block == 0 && tid == 0) P.stops[b] = 0;
+    if (tid < cols && block * cols + tid < D) *last_reading_out = handed_over(0);
     return;
   }
   const int lane = tid % kWave;
@@ -254,7 +275,7 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
   // Whether the sequence ends in chunk c.  A wave asks after the chunk's last
   // barrier, and what a faster one may have set by then is a later chunk's.
   // (A relaxed load: a volatile one waits for the wave's stores.  Once a chunk:
-  // asked for every token by the store waves it took 10 us of 100 at B = 16,
+  // asked for every token by the store waves it took 10 us of 98 at B = 16,
   // T = 128, N = 256, D = 128.)
   auto stops_in = [&](int64_t c) __attribute__((always_inline)) {
     return (__hip_atomic_load(stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >> kDrShift) <=
@@ -503,7 +524,7 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
             now_a = next_a;
             const float reading = last_reading();
             keep = g == (u + kRrGroups - 1) % kRrGroups ? reading : keep;
-            if (u == 0 && j0 > 0 && t < T && d < D) *out = keep;
+            if (u == 0 && j0 > 0 && t < T && d < D) *out = done_reading(keep);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               old_rw[i] = rw[i];
@@ -519,7 +540,7 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
           // results are the next kernel's
           const float before = last_reading();
           keep = g == kRrGroups - 1 ? before : keep;
-          if (j0 > 0 && t < T && d < D) *out = keep;
+          if (j0 > 0 && t < T && d < D) *out = done_reading(keep);
           const int first = stopped ? 0 : __builtin_ctz(dense);
           for (int u = 0; u < first; ++u) {
             const uint2 e = entry(pw + u * Rec::kBytes);
@@ -574,7 +595,7 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
       // the chunk's last reading and its last store
       const float reading = last_reading();
       keep = g == kRrGroups - 1 ? reading : keep;
-      if (t < T && d < D) *out = keep;
+      if (t < T && d < D) *out = done_reading(keep);
       if (!STATES) __syncthreads();
       if (stopped) break;
     }
@@ -586,7 +607,6 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
   if (bad) *redo = 1;
   __syncthreads();   // what the store waves wrote is out, too
   const int64_t end = *stop < T ? *stop : T;
-  if (block == 0 && tid == 0 && T > 0) P.stops[b] = end;
   if (*redo) {
     if (__ballot(bad)) {
       redo_columns<STATES>(P, lds + wave * table_bytes + col * 4, b, d0 + wave * kRrCols + col, g,
@@ -594,7 +614,10 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
     }
     __syncthreads();
   }
-  if (end < T) return;
+  if (end < T) {
+    if (tid < cols && d0 + tid < D) *last_reading_out = handed_over(end);
+    return;
+  }
   if (!P.final_memory) return;
   float* const out = P.final_memory + b * N * static_cast<int64_t>(D);
   const int at_once = static_cast<int>(blockDim.x) / per_row;
@@ -707,9 +730,12 @@ __global__ __launch_bounds__(kRecThreads) void dense_recurrence_kernel(RecParams
   const int col = lane / kRecGroups;
   const int g = lane % kRecGroups;
   const int N = P.slots, D = P.width;
-  const int64_t start = P.all_dense ? 0 : P.stops[b];
+  // its columns hold the same number; the same in every lane of the wave
+  const int64_t start =
+      P.all_dense ? 0
+                  : handed_over_at(P.readings[((b + 1) * P.time - 1) * D + cb * kRecCols]);
+  if (start < 0) return;
   const int64_t T = P.time - start;
-  if (!P.all_dense && T <= 0) return;
   const int64_t first = b * P.time + start;   // of the tokens, over the batch
   const int d = cb * kRecCols + col;
   const bool col_ok = d < D;
@@ -904,9 +930,9 @@ int32_t launch_recurrence(RecParams& P, hipStream_t s) {
   int nw = (P.width + kRrCols - 1) / kRrCols;
   nw = nw > kRrWaves ? kRrWaves : nw;
   // with per-token memories two waves where four would leave CUs idle, for a
-  // CU writes 64 bytes a cycle: 98 us against 109 at B = 16, T = 128, N = 256,
+  // CU writes 64 bytes a cycle: 87 us against 102 at B = 16, T = 128, N = 256,
   // D = 128; where four fill the chip their 128-byte rows are the better ones
-  // (265 us against 284 at B = 64, T = 16, N = 1024, D = 256)
+  // (241 us against 266 at B = 64, T = 16, N = 1024, D = 256)
   if (STATES && nw > 2 && P.batch * ((P.width + nw * kRrCols - 1) / (nw * kRrCols)) < kCus) nw = 2;
   while (nw > 1 && bytes(nw) > kRrLds) --nw;
   const int lds = bytes(nw);
@@ -935,11 +961,6 @@ int32_t launch_recurrence_slots(RecParams& P, hipStream_t s) {
 using namespace cowsdm_impl;
 
 extern "C" int32_t cowsdm_recurrence_forward(const cowsdm_recurrence_t* r, void* stream) {
-  return cowsdm_recurrence_forward_stops(r, nullptr, stream);
-}
-
-extern "C" int32_t cowsdm_recurrence_forward_stops(const cowsdm_recurrence_t* r, int64_t* stops,
-                                                   void* stream) {
   if (!r) return fail(COWSDM_EARG, "recurrence: null argument");
   if (r->batch < 0 || r->time < 0 || r->slots <= 0 || r->width <= 0) {
     return fail(COWSDM_EARG, "recurrence: invalid sizes");
@@ -970,7 +991,6 @@ extern "C" int32_t cowsdm_recurrence_forward_stops(const cowsdm_recurrence_t* r,
   P.eg = r->erase_gate;
   P.flg = r->forget_log_gate;
   P.rr = r->read_routes;
-  P.stops = stops;
   P.readings = r->readings;
   P.states = r->states;
   P.final_memory = r->final_memory;
@@ -987,9 +1007,9 @@ extern "C" int32_t cowsdm_recurrence_forward_stops(const cowsdm_recurrence_t* r,
   // either kernel for all of N <= 64 one of these sides loses a third or more.
   // And the sparse sequences' launch, at most 16 waves to 16 columns, has to
   // stay below 2^32 threads.
-  // Without a place for where sequences are handed over, and for their memory
-  // there, none is.
-  P.all_dense = !P.stops || (!P.states && !P.final_memory) ||
+  // A sequence is handed over with its memory in one of the outputs and the
+  // token's number in the low bits of a float.
+  P.all_dense = (!P.states && !P.final_memory) || P.time >= kDrMaxTime ||
                 (P.slots <= kWave && P.batch * P.width < 4096) ||
                 (P.batch + kXcds - 1) * ((P.width + 15) / 16) >= (int64_t{1} << 22);
   if (P.all_dense) return launch_dense_sequences(P, s);

@@ -6,7 +6,7 @@ recurrence the reference runs for training and prefill
 (sdm.py:162-172), which scatters product-key routes into the dense vectors
 the recurrence takes.
 
-Kernels: ``cowsdm_recurrence_forward_stops`` and ``cowsdm_dense_routes``
+Kernels: ``cowsdm_recurrence_forward`` and ``cowsdm_dense_routes``
 (csrc/recurrence.hip), and for the prefill, which holds the sparse routes,
 ``cowsdm_route_recurrence_forward`` (csrc/route_recurrence.hip).  Float32 only; there is no CPU path (the reference
 falls back to its serial torch loop off CUDA, this module raises).
@@ -123,9 +123,8 @@ def sdm_recurrence(initial_memory: torch.Tensor, write_routes: torch.Tensor,
     r.readings = readings.data_ptr()
     r.states = states.data_ptr() if states is not None else None
     r.final_memory = final.data_ptr()
-    stops = torch.empty(batch, device=device, dtype=torch.int64)
-    nat.check(nat.lib().cowsdm_recurrence_forward_stops(
-        r, stops.data_ptr(), nat.stream_handle(device)), "cowsdm_recurrence_forward_stops")
+    nat.check(nat.lib().cowsdm_recurrence_forward(r, nat.stream_handle(device)),
+              "cowsdm_recurrence_forward")
     if return_states:
         return readings, final, states
     return readings, final

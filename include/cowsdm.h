@@ -735,15 +735,8 @@ typedef struct cowsdm_recurrence {
 } cowsdm_recurrence_t;
 
 /* Runs the recurrence of cowsdm_recurrence_t; COWSDM_ELIMIT for N > 1024
- * (the reference's "at most 1,024 slots").  Every token is summed over all of
- * its N slots. */
+ * (the reference's "at most 1,024 slots"). */
 int32_t cowsdm_recurrence_forward(const cowsdm_recurrence_t* recurrence, void* stream);
-
-/* The same with `stops`, [B] words of scratch: tokens with few nonzero routes
- * are summed over those, a sequence's tokens up to its first one with many.
- * (Without states and final_memory as cowsdm_recurrence_forward.) */
-int32_t cowsdm_recurrence_forward_stops(const cowsdm_recurrence_t* recurrence, int64_t* stops,
-                                        void* stream);
 
 /* One SDM layer's token-serial recurrence over sparse routes (float32,
  * device, contiguous): the recurrence of cowsdm_recurrence_t for routes that
