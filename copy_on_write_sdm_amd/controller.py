@@ -515,7 +515,7 @@ class ControllerDecodeGraph:
     def _record(self, stream: int, structs) -> torch.Tensor:
         """Per layer: prepare with the routes, the step, finish with the
         residual add.  Without a tail between layers a layer's finish and the
-        next layer's prepare are one call (one launch at sqrt(N) <= 64)."""
+        next layer's prepare are one call (one launch where that is the faster way)."""
 
         lib = nat.lib()
         x = self.tokens.contiguous()

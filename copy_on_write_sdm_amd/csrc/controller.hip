@@ -79,7 +79,7 @@ struct CtlParams {
   int ld;                     // floats from one token's row in LDS to the next
 };
 
-// The routes the prepare kernel selects itself (sqrt(N) <= 64): every
+// The routes the prepare kernel selects itself (prepare_selects): every
 // token's read and write route rows, one wave per row.
 struct CtlRoutes {
   int root, read_sub, read_k, write_sub, write_k;

@@ -669,10 +669,10 @@ int32_t cowsdm_controller_finish(const cowsdm_controller_t* controller,
 /* cowsdm_controller_prepare followed by the product-key routes of every
  * token's read and write keys (sdm.py:96-159, as
  * _prepare_faithful_sdm_step calls them, inference.py:479-488), in one
- * launch when sqrt(slots) <= 64: read_weights/read_indices
- * [batch * heads, min(reads, min(reads, sqrt N)^2)], the write routes
- * likewise; larger tables fall back to the three separate launches.  The
- * routes equal cowsdm_product_key_routes' bit for bit; reads and writes
+ * launch where that is the faster way (sqrt(slots) <= 64, up to 4,096 route
+ * rows, a projection of few rounds) and in three elsewhere:
+ * read_weights/read_indices [batch * heads, min(reads, min(reads, sqrt N)^2)],
+ * the write routes likewise.  The routes equal cowsdm_product_key_routes' bit for bit; reads and writes
  * take its `selected` checks.  No single counterpart in the reference: it
  * is the fusion of the calls above for a decode step's launch count. */
 int32_t cowsdm_controller_prepare_routes(
@@ -695,9 +695,8 @@ int32_t cowsdm_controller_finish_residual(const cowsdm_controller_t* controller,
  * on out_sum: the layer stack's per-token walk (inference.py:655-661) for
  * a caller with nothing between the layers (the reference's stack puts an
  * MLP there, inference.py:661, and takes the two calls), in one launch
- * when the next layer's
- * sqrt(slots) <= 64 (its tokens' inputs stay on chip between the two), else
- * in the two launches.  The layers share their width.  Every output equals
+ * where the next layer's prepare selects its routes in its own (its tokens'
+ * inputs stay on chip between the two), else as the two calls.  The layers share their width.  Every output equals
  * the two calls' bit for bit.  No single counterpart in the reference. */
 int32_t cowsdm_controller_finish_prepare_routes(
     const cowsdm_controller_t* controller, const float* normalized, const float* reading,
