@@ -672,9 +672,10 @@ int32_t cowsdm_controller_finish(const cowsdm_controller_t* controller,
  * launch where that is the faster way (sqrt(slots) <= 64, up to 4,096 route
  * rows, a projection of few rounds) and in three elsewhere:
  * read_weights/read_indices [batch * heads, min(reads, min(reads, sqrt N)^2)],
- * the write routes likewise.  The routes equal cowsdm_product_key_routes' bit for bit; reads and writes
- * take its `selected` checks.  No single counterpart in the reference: it
- * is the fusion of the calls above for a decode step's launch count. */
+ * the write routes likewise.  The routes equal cowsdm_product_key_routes' bit
+ * for bit; reads and writes take its `selected` checks.  No single counterpart
+ * in the reference: it is the fusion of the calls above for a decode step's
+ * launch count. */
 int32_t cowsdm_controller_prepare_routes(
     const cowsdm_controller_t* controller, const float* tokens, int64_t batch,
     float* normalized, float* read_keys, float* write_keys, float* values, float* input_gate,
