@@ -184,9 +184,15 @@ __device__ __forceinline__ void redo_columns(const RecParams& P, char* mine, int
         }
       }
     }
-    // every row of these columns is NaN, and so is what follows; their
+    // once every row of these columns is NaN, so is what follows; their
     // readings are already
-    if (!STATES && __ballot(bad && delta == delta) == 0) break;
+    if (__ballot(bad && delta == delta) == 0) {
+      float* to = P.states + (bt + 1) * N * static_cast<int64_t>(D) + d;
+      for (int64_t n = g; STATES && bad && n < (end - 1 - t) * N; n += kRrGroups) {
+        to[n * D] = __builtin_nanf("");
+      }
+      break;
+    }
   }
   if (!STATES && end < T) {
     for (int n = g; n < N; n += kRrGroups) {
