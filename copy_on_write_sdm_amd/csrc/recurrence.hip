@@ -237,10 +237,10 @@ __global__ __launch_bounds__(kDrThreads + (STATES ? kDrStoreThreads : 0)) void r
     return reinterpret_cast<Vec*>(lds + (c / kRrCols) * table_bytes + n * kRrRowBytes +
                                   (c % kRrCols) * 4);
   };
-  // 0 or NaN per column: whether the initial memory holds a non-finite value
-  // the sequence's first dense token, set by the compute waves in its chunk
-  // (all the same value), for all others at the end of that chunk; whether
-  // some columns are taken again
+  // `poison`, 0 or NaN per column: whether the initial memory holds a value
+  // that is not finite.  `stop`: the sequence's first dense token, set by the
+  // compute waves in its chunk (all the same value), for all others at the end
+  // of that chunk.  `redo`: whether some columns are taken again.
   int64_t* const stop = reinterpret_cast<int64_t*>(poison + cols);
   int* const redo = reinterpret_cast<int*>(stop + 1);
   if (tid < cols) poison[tid] = 0.0f;
